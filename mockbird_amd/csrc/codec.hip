@@ -78,7 +78,7 @@ struct CodecState {
   int32_t* pos = nullptr;   // [4][max_voices]: the next absolute position of each stage
   int32_t* nrow = nullptr;  // [4][max_voices]: positions per frame of each stage
   float *acc = nullptr, *x = nullptr, *h = nullptr, *qkv = nullptr, *att = nullptr,
-        *ffn = nullptr, *wide = nullptr;
+        *ffn = nullptr, *wide = nullptr, *part = nullptr;
   int32_t* frame = nullptr;  // the frame a decode call is at (device counter)
   std::vector<void*> owned;
   // one captured frame of mb_codec_decode_dev and what it was captured for
@@ -417,7 +417,7 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
       };
       if ((rc = qkv_proj()) ||
           (rc = launch_window_attention(ctx, ring, B, n, cs.qkv, dense_rows(3 * kD, n), pos, nrow,
-                                        cs.att, dense_rows(kD, n))) ||
+                                        cs.att, dense_rows(kD, n), cs.part)) ||
           (rc = x3 ? launch_gemm_x3(ctx, EPI_SCALE_ADD, cs.att, kD, w.o_x, kD, kD, w.s1, cs.x, kD,
                                       M, nullptr, nullptr)
                      : launch_gemm(ctx, EPI_SCALE_ADD, cs.att, kD, w.o, kD, kD, w.s1, cs.x, kD, M)) ||
@@ -510,10 +510,11 @@ extern "C" int mb_codec_init(mb_ctx* ctx, const mb_codec_config* cfg) {
   cs->att = (float*)dev_alloc(ctx, *cs, (size_t)rows * kD * 4);
   cs->ffn = (float*)dev_alloc(ctx, *cs, (size_t)rows * kFfn * 4);
   cs->wide = (float*)dev_alloc(ctx, *cs, (size_t)rows * kRvqOut * 4);
+  cs->part = (float*)dev_alloc(ctx, *cs, kWindowPartFloats * 4);
   for (void* p : {cs->ring_k, cs->ring_v, (void*)cs->slot_pos, (void*)cs->pos, (void*)cs->nrow,
                   (void*)cs->frame,
                   (void*)cs->acc, (void*)cs->x, (void*)cs->h, (void*)cs->qkv,
-                  (void*)cs->att, (void*)cs->ffn, (void*)cs->wide})
+                  (void*)cs->att, (void*)cs->ffn, (void*)cs->wide, (void*)cs->part})
     if (!p) {
       codec_free(ctx);
       return fail(ctx, MB_ERR_NOMEM, "codec rings and buffers for %d voices", V);

@@ -294,9 +294,13 @@ int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_
 // (the codec's stages), out of the causal windowed rule: qkv holds the fused
 // fp32 rows (q | k | v, ring.heads x 64 each); every row is roped and written
 // into the ring as launch_ring_write writes it, then its query attends.
+// part: room for kWindowPartFloats floats lets few sequences' windows be
+// shared between workgroups; null keeps one workgroup per (sequence, head).
+constexpr size_t kWindowPartFloats = (size_t)256 * 32 * 68;
 int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                             const float* qkv, const Rows& qkv_rows, const int32_t* pos0,
-                            const int32_t* n_rows, float* out, const Rows& out_rows);
+                            const int32_t* n_rows, float* out, const Rows& out_rows,
+                            float* part = nullptr);
 int launch_fill_i32(mb_ctx* ctx, int32_t* p, int64_t n, int32_t value);
 int launch_fill_kv(mb_ctx* ctx, void* p, int64_t n, float value);
 

@@ -654,14 +654,25 @@ __global__ __launch_bounds__(256) void k_flash_f32(
 //    products keep about 16 bits (the scores and weights agree with the fp32
 //    path to ~1e-5 relative) at an eighth of the fp32 MFMA time.
 // Partials (max, sum, 64 dims per query) fold across the waves through LDS.
+// SPLIT: gridDim.z workgroups share one window, and each leaves its folded
+// state in `part` (k_window_merge adds them up).  Where a launch has few
+// units, the bound is one workgroup's chain of dependent groups, not the
+// memory: a voice's stage-4 layer (3280 slots, fp32) took 77.8 us on 4
+// workgroups, 12.7 + 4.9 us on 64 and the merge.
 // Liveness is the window rule: slot position p (empty slots never live) is
 // visible to a query at cur iff 0 <= cur - p < W.
-template <bool KV_BF16, int QB, int NW>
+constexpr int kWindowWaves = 8;          // waves per workgroup
+constexpr int kWindowSplitBlocks = 256;  // workgroups of a split launch at most (one per CU)
+constexpr int WPART = HD + 4;  // floats of a SPLIT state: 64 sums, max (log2 units), denominator
+static_assert((size_t)kWindowSplitBlocks * 32 * WPART <= kWindowPartFloats, "split states");
+
+template <bool KV_BF16, int QB, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void k_attn_window(
     const float* __restrict__ qkv, Rows qkv_rows, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ n_rows, void* __restrict__ ring_k, void* __restrict__ ring_v,
     int32_t* __restrict__ slot_pos, int64_t ring_seq_stride, int C, int W, int wrap,
-    const float2* __restrict__ rope_tab, float* __restrict__ out, Rows out_rows) {
+    const float2* __restrict__ rope_tab, float* __restrict__ out, Rows out_rows,
+    float* __restrict__ part) {
   constexpr int NQ = 16 * QB;
   __shared__ float red_ml[NW][2][NQ];        // per wave: max (log2 units), sum
   __shared__ float red_acc[NW][NQ][HD + 1];  // per wave: unnormalised output
@@ -669,6 +680,10 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int qc = lane & 15, g = lane >> 4;
   const int h = blockIdx.x, b = blockIdx.y;
+  // SPLIT: workgroup z of gridDim.z takes the groups g0, g0 + step, ... of
+  // its waves (the unsplit workgroup's numbering with gridDim.z * NW waves)
+  const int g0 = SPLIT ? (int)blockIdx.z * NW + wave : wave;
+  const int step = SPLIT ? (int)gridDim.z * NW : NW;
   const int n = n_rows[b];
   const int64_t p0 = pos0[b];
   const int64_t end64 = p0 + n;
@@ -723,8 +738,8 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
   // after the barrier.
   Raw cur, nxt;
   bool early = false;
-  if (wave < groups && p0 >= 0) {
-    const int lo = wave * 16, hi = min(lo + 16, kv_end);
+  if (g0 < groups && p0 >= 0) {
+    const int lo = g0 * 16, hi = min(lo + 16, kv_end);
     const int wr0 = n > C ? n - C : 0;
     const int len = n - wr0;
     bool hit = true;
@@ -737,7 +752,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
       hit = end <= C ? (start < hi && lo < end) : (start < hi || lo < end - C);
     }
     early = !hit;
-    if (early) load_group(wave, cur);
+    if (early) load_group(g0, cur);
   }
 
   // The chunk's rows enter the ring first, as k_ring_write writes them but
@@ -769,10 +784,15 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
         }
         if (!(n > C && r < n - C)) {
           const int slot = wrap ? (int)(p64 % C) : (int)p64;
-          const int64_t koff = (int64_t)b * ring_seq_stride + ((int64_t)h * C + slot) * HD + d0;
-          store8<KV_BF16>(ring_k, koff, ko);
-          store8<KV_BF16>(ring_v, koff, vv);
-          if (d0 == 0) slot_pos[(int64_t)b * C + slot] = pos;
+          // SPLIT: a row is written by the workgroup that reads its slot
+          // (slots of live rows are below kv_end), so no workgroup waits for
+          // another's stores
+          if (!SPLIT || (slot >> 4) % step / NW == (int)blockIdx.z) {
+            const int64_t koff = (int64_t)b * ring_seq_stride + ((int64_t)h * C + slot) * HD + d0;
+            store8<KV_BF16>(ring_k, koff, ko);
+            store8<KV_BF16>(ring_v, koff, vv);
+            if (d0 == 0) slot_pos[(int64_t)b * C + slot] = pos;
+          }
         }
       } else {
 #pragma unroll
@@ -786,7 +806,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
   __syncthreads();  // the rows are in the ring and q in LDS for every wave
 
   // the wave's first group is in flight while q is split
-  if (wave < groups && !early) load_group(wave, cur);
+  if (g0 < groups && !early) load_group(g0, cur);
   // Positions relative to the sequence's first query, clamped so the window
   // test is one unsigned compare; an empty slot and a query past n are
   // outside every window.
@@ -831,8 +851,8 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
     l[qb] = 0.f;
   }
 
-  for (int gi = wave; gi < groups; gi += NW) {
-    load_group(gi + NW < groups ? gi + NW : gi, nxt);  // past the wave's last group: a reload, unused
+  for (int gi = g0; gi < groups; gi += step) {
+    load_group(gi + step < groups ? gi + step : gi, nxt);  // past the wave's last group: a reload, unused
     const int s0 = gi * 16;
     float kf[16];
     bf16x8_t kh[2];
@@ -968,32 +988,119 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
         o += wt * red_acc[w][qi][dim];
       }
     }
-    out[row_at(out_rows, b, qi) + h * HD + dim] = L > 0.f ? o / L : 0.f;
+    if constexpr (SPLIT) {
+      float* pp = part + (((int64_t)b * gridDim.x + h) * gridDim.z + blockIdx.z) * (NQ * WPART) +
+                  qi * WPART;
+      pp[dim] = o;
+      if (dim == 0) {
+        pp[HD] = M;
+        pp[HD + 1] = L;
+      }
+    } else {
+      out[row_at(out_rows, b, qi) + h * HD + dim] = L > 0.f ? o / L : 0.f;
+    }
   }
+}
+
+// Merges the SPLIT form's states: workgroup (head, sequence), thread (query,
+// 4 dims).  Every split's maximum and sum are loaded before the first use,
+// then the weighted rows.
+template <int QB, int S>
+__global__ __launch_bounds__(256 * QB) void k_window_merge(const float* __restrict__ part,
+                                                           const int32_t* __restrict__ n_rows,
+                                                           float* __restrict__ out, Rows out_rows) {
+  constexpr int NQ = 16 * QB;
+  const int h = blockIdx.x, b = blockIdx.y;
+  const int qi = threadIdx.x >> 4, dim = (threadIdx.x & 15) * 4;
+  const float* pp = part + ((int64_t)b * gridDim.x + h) * S * (NQ * WPART) + qi * WPART;
+  const int n = n_rows[b];  // rows past it have no state: what is loaded for them is not stored
+  float2 ml[S];
+  float4 o[S];
+#pragma unroll
+  for (int s = 0; s < S; s++) {
+    ml[s] = *(const float2*)(pp + s * (NQ * WPART) + HD);
+    o[s] = *(const float4*)(pp + s * (NQ * WPART) + dim);
+  }
+  float M = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < S; s++) M = fmaxf(M, ml[s].x);
+  float L = 0.f;
+  float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int s = 0; s < S; s++) {
+    const float wt = ml[s].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - M);
+    L += wt * ml[s].y;
+    r.x += wt * o[s].x; r.y += wt * o[s].y; r.z += wt * o[s].z; r.w += wt * o[s].w;
+  }
+  if (L > 0.f) {
+    r.x /= L; r.y /= L; r.z /= L; r.w /= L;
+  } else {
+    r = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (qi < n) *(float4*)(out + row_at(out_rows, b, qi) + h * HD + dim) = r;
+}
+
+// How many workgroups share a (sequence, head) window of `slots`: a power of
+// two up to 16 that keeps the launch within one workgroup per CU and leaves
+// every wave a 16-slot group.  With one workgroup per unit a voice's 4 heads
+// are 4 workgroups, each a chain of ~26 dependent groups per wave at 3280
+// slots.  Per 4-frame codec call on full windows, one workgroup -> this rule:
+// fp32 rings 1 / 8 / 32 voices 3213 -> 1884 / 3460 -> 2223 / 3791 -> 3251 us,
+// bf16 2222 -> 1735 / 2092 -> 1631 / 2591 -> 2444 us.  Two workgroups per CU
+// lost from 8 voices up (fp32 2362 / 3390 us at 8 / 32), as did splitting the
+// 64 voices that already fill the chip (4623 -> 4923 us); two groups per wave
+// cost a single voice 6 % (2002 us).
+int window_splits(int units, int slots) {
+  const int groups = (slots + 15) / 16;
+  int s = 1;
+  while (s < 16 && 2 * s * units <= kWindowSplitBlocks && groups >= 2 * s * kWindowWaves) s *= 2;
+  return s;
 }
 
 // Chunks of up to 32 consecutive rows per sequence (the codec's stages):
 // each row's K/V enters the ring and its query attends the window in one
-// launch; rows_max bounds n_rows.
+// launch; rows_max bounds n_rows.  `part` (kWindowPartFloats floats, or null)
+// lets a launch with few (sequence, head) units share each window between
+// workgroups, whose states a second launch merges.
 int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                             const float* qkv, const Rows& qkv_rows, const int32_t* pos0,
-                            const int32_t* n_rows, float* out, const Rows& out_rows) {
+                            const int32_t* n_rows, float* out, const Rows& out_rows, float* part) {
   if (rows_max < 1 || rows_max > 32)
     return fail(ctx, MB_ERR_ARG, "window attention takes 1..32 rows per sequence, not %d", rows_max);
   if (B > 65535) return fail(ctx, MB_ERR_ARG, "at most 65535 sequences per call");
   if (B == 0) return MB_OK;
-  constexpr int NW = 8;
-  const dim3 grid((unsigned)ring.heads, (unsigned)B);
-#define MB_WIN(BF, QB)                                                                            \
-  hipLaunchKernelGGL((k_attn_window<BF, QB, NW>), grid, dim3(64 * NW), 0, ctx->stream, qkv,      \
-                     qkv_rows, pos0, n_rows, ring.k, ring.v, ring.sp, ring.seq_stride, ring.C,   \
-                     ring.window, ring.wrap, ctx->rope_tab, out, out_rows)
-  if (ring.bf16) {
-    if (rows_max <= 16) MB_WIN(true, 1); else MB_WIN(true, 2);
-  } else {
-    if (rows_max <= 16) MB_WIN(false, 1); else MB_WIN(false, 2);
-  }
-#undef MB_WIN
+  constexpr int NW = kWindowWaves;
+  const int S = part ? window_splits(ring.heads * B, ring.C) : 1;
+  const dim3 grid((unsigned)ring.heads, (unsigned)B, (unsigned)S);
+  auto go = [&](auto bf_, auto qb_, auto split_) {
+    constexpr bool BF = decltype(bf_)::value, SP = decltype(split_)::value;
+    constexpr int QB = decltype(qb_)::value;
+    hipLaunchKernelGGL((k_attn_window<BF, QB, NW, SP>), grid, dim3(64 * NW), 0, ctx->stream, qkv,
+                       qkv_rows, pos0, n_rows, ring.k, ring.v, ring.sp, ring.seq_stride, ring.C,
+                       ring.window, ring.wrap, ctx->rope_tab, out, out_rows, part);
+  };
+  auto merge = [&](auto qb_, auto s_) {
+    constexpr int QB = decltype(qb_)::value;
+    hipLaunchKernelGGL((k_window_merge<QB, decltype(s_)::value>),
+                       dim3((unsigned)ring.heads, (unsigned)B), dim3(256 * QB), 0, ctx->stream,
+                       part, n_rows, out, out_rows);
+  };
+  using std::integral_constant;
+  auto all = [&](auto qb_) {
+    if (S == 1) {
+      if (ring.bf16) go(std::true_type{}, qb_, std::false_type{});
+      else go(std::false_type{}, qb_, std::false_type{});
+      return;
+    }
+    if (ring.bf16) go(std::true_type{}, qb_, std::true_type{});
+    else go(std::false_type{}, qb_, std::true_type{});
+    if (S == 2) merge(qb_, integral_constant<int, 2>{});
+    else if (S == 4) merge(qb_, integral_constant<int, 4>{});
+    else if (S == 8) merge(qb_, integral_constant<int, 8>{});
+    else merge(qb_, integral_constant<int, 16>{});
+  };
+  if (rows_max <= 16) all(integral_constant<int, 1>{});
+  else all(integral_constant<int, 2>{});
   MB_HIP(ctx, hipGetLastError());
   return MB_OK;
 }

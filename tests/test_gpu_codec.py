@@ -160,6 +160,28 @@ def test_codec_full_size_long_run(B, kv, frames):
     say(f"  max error / scale over {len(watch)} voices: {worst:.2e}")
 
 
+@pytest.mark.parametrize("B,kv", [(1, mb.MB_KV_F32), (3, mb.MB_KV_BF16), (17, mb.MB_KV_F32)])
+def test_codec_shared_windows(B, kv):
+    """Few voices: each (voice, head) window is shared between workgroups and
+    merged.  Windows just past 2, 2, 4 and 8 workgroups' worth of 16-slot
+    groups (8 waves each), decoded from empty rings (workgroups without a
+    group) until stages 2-4 wrap; 17 voices split the long windows only."""
+    say(f"codec shared windows, {B} voices, kv={kv}")
+    layers, context = (1, 1, 1, 1), (245, 260, 520, 1030)
+    watch = sorted({0, B // 2, B - 1})
+    w = synth.codec_weights(layers, seed=23)
+    codes = synth.codec_codes(24, 40, B)
+    ora = oracle.CodecOracle(w, len(watch), layers, context, kv_bf16=(kv == mb.MB_KV_BF16))
+    want = ora.decode(np.ascontiguousarray(codes[:, watch]))
+    with _ctx() as ctx:
+        ctx.upload_all(w)
+        ctx.codec_init(B, layers, context, kv_dtype=kv)
+        got = np.concatenate([ctx.codec_decode(codes[f:f + 10]) for f in range(0, 40, 10)], axis=2)
+    rel = 2e-5 if kv == mb.MB_KV_F32 else 1e-3
+    for i, b in enumerate(watch):
+        say(f"  voice {b}: {_close(got[b], want[i], rel, f'voice {b}'):.2e}")
+
+
 def test_codec_argument_errors():
     say("codec argument errors")
     with _ctx() as ctx:
