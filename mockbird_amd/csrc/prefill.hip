@@ -2,14 +2,11 @@
 // matrix is ever materialised (the reference writes [12, S, S] scores and
 // probabilities, kernels-batch.ts:246-350, and caps S at 256, prefill.ts:136).
 //
-// One workgroup = 64 query rows of one (sequence, head); each of its 4 waves
-// owns 16 query columns.  The kernel computes S^T = K Q^T so that the
-// accumulator tile (lane l holds rows (l/16)*4 + j, column l%16) is already
-// the B operand of the next MFMA: for bf16 that is v_mfma_f32_16x16x16_bf16
-// (B lane l = rows (l/16)*4 + j, column l%16), so P^T goes from the softmax
-// straight into O^T += V^T P^T without an LDS round trip.  Per 64-slot K/V
-// tile a wave issues 8 (bf16: 16x16x32) or 64 (fp32: 16x16x4) MFMAs for the
-// scores and 16 / 64 for P V.
+// A wave owns 16 or 32 query columns of one (sequence, head).  The kernels
+// compute S^T = K Q^T so that the accumulator tile (lane l holds rows
+// (l/16)*4 + j, column l%16) is already half of the B operand of the next
+// v_mfma_f32_16x16x32_bf16 (the order of its k values is free), so P^T goes
+// from the softmax straight into O^T += V^T P^T without an LDS round trip.
 //
 // Queries: row r of sequence b sits at position cur = pos0[b] + r and sees
 // the ring slots whose stored position p satisfies 0 <= cur - p < C (the
@@ -29,9 +26,8 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int KT = 64;    // slots per K/V tile
-constexpr int QT = 64;    // query rows per workgroup
-constexpr int FPAD = 68;  // fp32 LDS row stride (272 B)
+constexpr int KT = 64;    // slots per K/V tile of the bf16 kernel
+constexpr int QT = 64;    // query rows per workgroup of the fp32-query kernel
 
 // Workgroup -> (sequence, head, query tile).  Query tile t of a causal
 // prefill costs about t + 1 K/V tiles, so the work is numbered latest tile
@@ -67,11 +63,6 @@ __device__ __forceinline__ void work_item(int& b, int& h, int& qtile, int nxcd, 
   const uint32_t hb = g % pairs;
   h = (int)(hb % gridDim.y);
   b = (int)(hb / gridDim.y);
-}
-
-__device__ __forceinline__ bool live_slot(int32_t p, int64_t cur, int C) {
-  const int64_t d = cur - p;
-  return p >= 0 && d >= 0 && d < C;
 }
 
 
@@ -498,132 +489,282 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
 }
 #undef MB_WAIT_VMCNT
 
-// ---------------------------------------------------------------- fp32 MMA
+// ------------------------------------------------------------ fp32 queries
 
-// Q fp32 [B][rows_max][768] (roped), K/V fp32 or bf16 ring (widened exactly
-// into LDS), fp32 output, v_mfma_f32_16x16x4f32.  The score MMA's k index
-// (0..3 per instruction, 16 instructions) is mapped to dim grp*16 + kc so a
-// lane reads 16 consecutive dims of its K row and of its Q row.  In P V the
-// instruction (sb, j) sums over k = grp, i.e. over slots sb*16 + grp*4 + j,
-// which is exactly the score element the lane already holds.
+// Three bf16 planes of a float: x = h + m + l exactly.  Cutting the low 16
+// bits leaves 8 significant bits, the remainder (exact) has at most 16, and
+// cutting that one leaves at most 8: three bf16 numbers.  (Overflow cannot
+// happen, as rounding to bf16 could; below 2^-110 the low plane may be
+// denormal.)  Eight values at a time, packed as MFMA operands.
+struct Planes {
+  bf16x8_t p[3];
+};
+__device__ __forceinline__ Planes split3(const float (&v)[8]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t a = __float_as_uint(v[2 * i]), b = __float_as_uint(v[2 * i + 1]);
+    w[0][i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    const float ra = v[2 * i] - __uint_as_float(a & 0xffff0000u);
+    const float rb = v[2 * i + 1] - __uint_as_float(b & 0xffff0000u);
+    const uint32_t ma = __float_as_uint(ra), mb = __float_as_uint(rb);
+    w[1][i] = __builtin_amdgcn_perm(mb, ma, 0x07060302u);
+    const float la = ra - __uint_as_float(ma & 0xffff0000u);
+    const float lb = rb - __uint_as_float(mb & 0xffff0000u);
+    w[2][i] = __builtin_amdgcn_perm(__float_as_uint(lb), __float_as_uint(la), 0x07060302u);
+  }
+  Planes r;
+#pragma unroll
+  for (int k = 0; k < 3; k++)
+    r.p[k] = __builtin_bit_cast(bf16x8_t, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
+  return r;
+}
+
+// f(i, j) for the plane pairs of a product of KP by three planes that are
+// kept, the smallest first: the planes' weights are 2^0, 2^-8, 2^-16, and
+// pairs beyond i + j = 2 are below 2^-24 of the product.
+template <int KP, class F>
+__device__ __forceinline__ void plane_pairs(F f) {
+  using std::integral_constant;
+  auto at = [&](auto i, auto j) {
+    if constexpr (decltype(i)::value < KP) f(i, j);
+  };
+  integral_constant<int, 0> c0;
+  integral_constant<int, 1> c1;
+  integral_constant<int, 2> c2;
+  at(c2, c0); at(c0, c2); at(c1, c1); at(c1, c0); at(c0, c1); at(c0, c0);
+}
+
+// Q fp32 [B][rows_max][768] (roped), K/V fp32 or bf16 ring, fp32 output: the
+// model's prompt passes.  Tile classes and online softmax are k_flash_bf16's;
+// every fp32 operand enters the bf16 matrix unit as three exact bf16 planes
+// (split3), so a 32-deep product of an fp32 and a bf16 operand is three
+// MFMAs of 16 cycles and one of two fp32 operands six, where
+// v_mfma_f32_16x16x4f32 takes eight of 32.  The fp32 matrix rate bounded the
+// kernel that used it.  The error against float64 is no larger than with fp32
+// products (1 x 281 rows, fp32 ring 2.5e-7 -> 2.3e-7 relative; bf16 ring
+// 3.3e-7 -> 2.8e-7): the sums are fp32 either way, in fewer roundings.
+//
+// A workgroup is 64 query rows of one (sequence, head), 16 per wave.  K/V
+// tiles of KS slots pass through registers into one of two LDS buffers (fp32
+// ones split on the way, once per workgroup), the next tile's loads in flight
+// under the current tile; one barrier per tile.  KS is 64 for bf16 rings and
+// 32 for fp32 ones, whose three planes fill the same 48 KB twice over; 64
+// fp32 slots (one workgroup per CU) took 98 us against 72 at 16 x 512 rows.
+// Also slower: 32 rows per wave (1 x 281 / 16 x 512 / 48 x 64..400 rows with
+// the ring write, fp32 ring 22.1 / 74.0 / 99.8 us against 17.5 / 71.6 / 92.8,
+// bf16 15.8 / 51.0 / 70.4 against 12.7 / 48.4 / 63.5: fewer workgroups, more
+// registers), two waves per workgroup (20.3 / 96.3 / 121.1 us, fp32), and
+// k_flash_bf16's snake order (equal).  With the fp32 MFMA kernel the same
+// calls took 28.3 / 109.3 / 130.6 us (fp32) and 29.1 / 106.2 / 121.7 (bf16).
 template <bool KV_BF16>
-__global__ __launch_bounds__(256) void k_flash_f32(
+__global__ __launch_bounds__(256, 3) void k_flash_x(
     const float* __restrict__ q, Rows q_rows, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ n_rows, const void* __restrict__ ring_k,
     const void* __restrict__ ring_v, const int32_t* __restrict__ slot_pos,
     int64_t ring_seq_stride, int C, int W, float* __restrict__ out, Rows out_rows) {
-  __shared__ float Ks[KT * FPAD];  // [slot][dim]
-  __shared__ float Vs[KT * FPAD];  // [slot][dim]
-  __shared__ int32_t Ps[KT];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int KP = KV_BF16 ? 1 : 3;   // planes of K and V
+  constexpr int KS = KV_BF16 ? 64 : 32;  // slots per tile
+  constexpr int IT = KS * 8 / 256;       // 8-dim chunks of K (and of V) per thread per tile
+  constexpr int U = KV_BF16 ? 1 : 2;     // 16-byte loads per chunk
+  constexpr int SB = KS / 16, CH = KS / 32;
+  __shared__ __align__(16) uint16_t Ks[2][KP][KS * HD];  // [slot][dim], chunks swizzled
+  __shared__ __align__(16) uint16_t Vs[2][KP][KS * HD];
+  __shared__ __align__(16) int32_t Ps[2][KS];            // stored position per slot
+  __shared__ __align__(16) int32_t Rl[4][KS];           // per wave: relative positions
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qcol = lane & 15, grp = lane >> 4;
   int b, h, qtile;
   work_item(b, h, qtile, 8, 0);
   const int n = n_rows[b];
-  if (qtile * QT >= n) return;
-  const int r = qtile * QT + wave * 16 + qcol;
-  const bool qvalid = r < n;
-  const int64_t cur = qvalid ? (int64_t)pos0[b] + r : -1;
+  if (qtile * QT >= n) return;  // uniform per workgroup, before any barrier
+  const int64_t p0 = pos0[b];
+  const int rw = qtile * QT + wave * 16;  // this wave's first query row
+  const bool wave_rows = rw < n;
   const int rlast = min(qtile * QT + QT, n) - 1;
-  const int64_t kv_end64 = (int64_t)pos0[b] + rlast + 1;
+  const int64_t kv_end64 = p0 + rlast + 1;
   const int kv_end = kv_end64 < C ? (int)kv_end64 : C;
 
-  float qv[16];
-  {
-    const float* qp = q + (qvalid ? row_at(q_rows, b, r) : 0) + h * HD + grp * 16;
-#pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      float4 t = qvalid ? *(const float4*)(qp + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-      qv[i] = t.x * 0.125f; qv[i + 1] = t.y * 0.125f; qv[i + 2] = t.z * 0.125f; qv[i + 3] = t.w * 0.125f;
-    }
-  }
   constexpr int E = KV_BF16 ? 2 : 4;
   const char* kb = (const char*)ring_k + ((int64_t)b * ring_seq_stride + (int64_t)h * C * HD) * E;
   const char* vb = (const char*)ring_v + ((int64_t)b * ring_seq_stride + (int64_t)h * C * HD) * E;
   const int32_t* sp = slot_pos + (int64_t)b * C;
+  // a tile in registers on its way to LDS
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t rk[IT][U], rv[IT][U];
+  int32_t rp = -1;
+  auto load = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const int it = tid + i * 256, slot = min(t0 + (it >> 3), kv_end - 1);
+      const int64_t off = ((int64_t)slot * HD + (it & 7) * 8) * E;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        rk[i][u] = *(const u32x4_t*)(kb + off + 16 * u);
+        rv[i][u] = *(const u32x4_t*)(vb + off + 16 * u);
+      }
+    }
+    if (tid < KS) rp = t0 + tid < kv_end ? sp[t0 + tid] : -1;
+  };
+  auto stash = [&](int bb) {
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+      const int it = tid + i * 256, e = swz(it >> 3, it & 7);
+      if constexpr (KV_BF16) {
+        *(u32x4_t*)&Ks[bb][0][e] = rk[i][0];
+        *(u32x4_t*)&Vs[bb][0][e] = rv[i][0];
+      } else {
+        float kf[8], vf[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          kf[j] = __uint_as_float(rk[i][j >> 2][j & 3]);
+          vf[j] = __uint_as_float(rv[i][j >> 2][j & 3]);
+        }
+        const Planes kp = split3(kf), vp = split3(vf);
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+          *(bf16x8_t*)&Ks[bb][p][e] = kp.p[p];
+          *(bf16x8_t*)&Vs[bb][p][e] = vp.p[p];
+        }
+      }
+    }
+    if (tid < KS) Ps[bb][tid] = rp;
+  };
+  load(0);
+
+  // B operands of the score MFMA: the planes of Q[row][32 kc + 8 grp + 0..7]
+  // times 1/sqrt(64) * log2(e) (one fp32 rounding), so the MFMAs yield the
+  // scores in log2 units
+  const int r = rw + qcol;
+  Planes qp[2];
+  {
+    const float* src = q + row_at(q_rows, b, min(r, n - 1)) + h * HD + grp * 8;
+#pragma unroll
+    for (int kc = 0; kc < 2; kc++) {
+      const float4 x = *(const float4*)(src + kc * 32), y = *(const float4*)(src + kc * 32 + 4);
+      const float v[8] = {x.x * kScoreLog2, x.y * kScoreLog2, x.z * kScoreLog2, x.w * kScoreLog2,
+                          y.x * kScoreLog2, y.y * kScoreLog2, y.z * kScoreLog2, y.w * kScoreLog2};
+      qp[kc] = split3(v);
+    }
+  }
+  // the window test in 32 bits, relative to the workgroup's first query (see
+  // k_flash_bf16)
+  const int64_t first = p0 + (int64_t)qtile * QT;
+  const int32_t ref = first < INT32_MAX ? (int32_t)first : INT32_MAX;
+  const int32_t ex = (int32_t)min(first - ref, (int64_t)1 << 30);
+  const int crel_lo = wave * 16 + ex, crel_hi = min(rw + 15, n - 1) - qtile * QT + ex;
+  const int crel = crel_lo + qcol;
 
   f32x4_t acc[4];
 #pragma unroll
   for (int d = 0; d < 4; d++) acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
+  float lsum = 0.f;                         // this lane's share of the column's weight sum
+  f32x4_t moff = f32x4_t{0.f, 0.f, 0.f, 0.f};  // -m (0 while m = -inf), where the scores start
+  float lim = -INFINITY;                    // rescale threshold on t = score - m
+  const int trow = grp * 4 + (qcol >> 2), tdim = (qcol & 3) * 4;
 
-  for (int t0 = 0; t0 < kv_end; t0 += KT) {
-    __syncthreads();
-    // stage K and V [slot][dim] as fp32; thread -> (slot, 8-dim chunk), 2 passes
+  auto compute = [&](int bb) {
+    const int32_t praw = Ps[bb][lane & (KS - 1)];
+    const int32_t rel_l = praw < 0 ? kRelEmpty : praw - ref;
+    if (__ballot(rel_l <= crel_hi) == 0) return;
+    const uint64_t partial =
+        ~(__ballot(rel_l <= crel_lo) & __ballot((uint32_t)crel_hi - (uint32_t)rel_l < (uint32_t)W));
+    f32x4_t s[SB];
 #pragma unroll
-    for (int pass = 0; pass < 2; pass++) {
-      const int sl = pass * 32 + (tid >> 3), dc = (tid & 7) * 8;
-      const int slot = t0 + sl;
-      float kf[8], vf[8];
-      if (slot < kv_end) {
-        load8<KV_BF16>(kb, (int64_t)slot * HD + dc, kf);
-        load8<KV_BF16>(vb, (int64_t)slot * HD + dc, vf);
-      } else {
+    for (int sb = 0; sb < SB; sb++) s[sb] = moff;
 #pragma unroll
-        for (int i = 0; i < 8; i++) kf[i] = vf[i] = 0.f;
-      }
-      *(float4*)(Ks + sl * FPAD + dc) = make_float4(kf[0], kf[1], kf[2], kf[3]);
-      *(float4*)(Ks + sl * FPAD + dc + 4) = make_float4(kf[4], kf[5], kf[6], kf[7]);
-      *(float4*)(Vs + sl * FPAD + dc) = make_float4(vf[0], vf[1], vf[2], vf[3]);
-      *(float4*)(Vs + sl * FPAD + dc + 4) = make_float4(vf[4], vf[5], vf[6], vf[7]);
+    for (int kc = 0; kc < 2; kc++) {
+      bf16x8_t ka[SB][KP];
+#pragma unroll
+      for (int sb = 0; sb < SB; sb++)
+#pragma unroll
+        for (int p = 0; p < KP; p++)
+          ka[sb][p] = *(const bf16x8_t*)&Ks[bb][p][swz(sb * 16 + qcol, kc * 4 + grp)];
+      plane_pairs<KP>([&](auto i, auto j) {
+#pragma unroll
+        for (int sb = 0; sb < SB; sb++)
+          s[sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[sb][i], qp[kc].p[j], s[sb], 0, 0, 0);
+      });
     }
-    if (tid < KT) Ps[tid] = (t0 + tid < kv_end) ? sp[t0 + tid] : -1;
-    __syncthreads();
-
-    float s[4][4];
-    float mt = -INFINITY;
+    if (partial) {  // uniform
+      Rl[wave][lane & (KS - 1)] = rel_l;
 #pragma unroll
-    for (int sb = 0; sb < 4; sb++) {
-      f32x4_t c = {0.f, 0.f, 0.f, 0.f};
-      const float* krow = Ks + (sb * 16 + qcol) * FPAD + grp * 16;
+      for (int sb = 0; sb < SB; sb++) {
+        if ((partial >> (16 * sb)) & 0xFFFFu) {  // uniform
+          const int4 pv = *(const int4*)&Rl[wave][sb * 16 + grp * 4];
+          const int32_t pj[4] = {pv.x, pv.y, pv.z, pv.w};
 #pragma unroll
-      for (int kc = 0; kc < 16; kc += 4) {
-        const float4 a4 = *(const float4*)(krow + kc);
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.x, qv[kc], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.y, qv[kc + 1], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.z, qv[kc + 2], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a4.w, qv[kc + 3], c, 0, 0, 0);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const bool ok = live_slot(Ps[sb * 16 + grp * 4 + j], cur, W);
-        s[sb][j] = ok ? c[j] : -INFINITY;
-        mt = fmaxf(mt, s[sb][j]);
+          for (int j = 0; j < 4; j++)
+            if ((uint32_t)(crel - pj[j]) >= (uint32_t)W) s[sb][j] = -INFINITY;
+        }
       }
     }
-    mt = col_max(mt);
-    const float mn = fmaxf(m, mt);
-    const float mu = mn == -INFINITY ? 0.f : mn;
-    const float scale = __expf(m - mu);
-    float ls = 0.f;
+    float xm = -INFINITY;
 #pragma unroll
-    for (int sb = 0; sb < 4; sb++)
+    for (int sb = 0; sb < SB; sb++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        s[sb][j] = __expf(s[sb][j] - mu);
-        ls += s[sb][j];
+      for (int j = 0; j < 4; j++) xm = fmaxf(xm, s[sb][j]);
+    if (__ballot(xm > lim)) {  // uniform
+      const float xt = col_max(xm);
+      if (xt > lim) {  // uniform per column
+        const float scale = lim == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(-xt);
+#pragma unroll
+        for (int d = 0; d < 4; d++) acc[d] *= scale;
+        lsum *= scale;
+#pragma unroll
+        for (int sb = 0; sb < SB; sb++) s[sb] -= xt;
+        moff -= xt;
+        lim = 8.f;
       }
-    l = l * scale + col_sum(ls);
-    m = mn;
+    }
 #pragma unroll
-    for (int d = 0; d < 4; d++) acc[d] *= scale;
+    for (int c = 0; c < CH; c++) {
+      float w[8];
 #pragma unroll
-    for (int sb = 0; sb < 4; sb++)
+      for (int e = 0; e < 8; e++) w[e] = __builtin_amdgcn_exp2f(s[2 * c + (e >> 2)][e & 3]);
+      lsum += ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
+      const Planes pp = split3(w);
+      bf16x8_t va[4][KP];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const float* vrow = Vs + (sb * 16 + grp * 4 + j) * FPAD + qcol;
+      for (int d = 0; d < 4; d++)
+#pragma unroll
+        for (int p = 0; p < KP; p++) {
+          const int dim = d * 16 + tdim;
+          const int e0 = swz(c * 32 + trow, dim >> 3) + (dim & 7);
+          const int e1 = swz(c * 32 + 16 + trow, dim >> 3) + (dim & 7);
+          const bf16x4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t*)&Vs[bb][p][e0]);
+          const bf16x4_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t*)&Vs[bb][p][e1]);
+          va[d][p] = bf16x8_t{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+        }
+      plane_pairs<KP>([&](auto i, auto j) {
 #pragma unroll
         for (int d = 0; d < 4; d++)
-          acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[d * 16], s[sb][j], acc[d], 0, 0, 0);
-      }
+          acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[d][i], pp.p[j], acc[d], 0, 0, 0);
+      });
+    }
+  };
+
+  stash(0);
+  if (KS < kv_end) load(KS);
+  int bb = 0;
+  for (int t0 = 0; t0 < kv_end; t0 += KS) {
+    // tile t0 is in LDS, and every wave is done with the buffer the next one
+    // goes to (read one tile ago)
+    __syncthreads();
+    if (wave_rows) compute(bb);
+    bb ^= 1;
+    if (t0 + KS < kv_end) {
+      stash(bb);
+      if (t0 + 2 * KS < kv_end) load(t0 + 2 * KS);
+    }
   }
-  if (!qvalid) return;
+  const float l = col_sum(lsum);
   const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (r >= n) return;
   float* op = out + row_at(out_rows, b, r) + h * HD;
 #pragma unroll
-  for (int d = 0; d < 4; d++)
-    *(float4*)(op + d * 16 + grp * 4) =
-        make_float4(acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv);
+  for (int d = 0; d < 4; d++) *(f32x4_t*)(op + d * 16 + grp * 4) = acc[d] * inv;
 }
 
 // ------------------------------------------------ short chunks, long windows
@@ -1115,7 +1256,6 @@ int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_
   if ((int64_t)((rows_max + QT - 1) / QT) * ring.heads * B >= INT32_MAX)
     return fail(ctx, MB_ERR_ARG, "too many query tiles in one prefill call");
   const unsigned nh = (unsigned)ring.heads;
-  dim3 grid((unsigned)((rows_max + QT - 1) / QT), nh, (unsigned)B);
   if (q_dtype == MB_DT_BF16)
     hipLaunchKernelGGL(k_flash_bf16<kFlashWaves>,
                        dim3((unsigned)((rows_max + BQ - 1) / BQ), nh, (unsigned)B),
@@ -1123,14 +1263,11 @@ int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_
                        pos0, n_rows, (const uint16_t*)ring.k, (const uint16_t*)ring.v, ring.sp,
                        ring.seq_stride, ring.C, ring.window, out, out_rows, ctx->xcds,
                        ctx->cus_per_xcd);
-  else if (ring.bf16)
-    hipLaunchKernelGGL(k_flash_f32<true>, grid, dim3(256), 0, ctx->stream, (const float*)q, q_rows,
-                       pos0, n_rows, ring.k, ring.v, ring.sp, ring.seq_stride, ring.C, ring.window,
-                       out, out_rows);
   else
-    hipLaunchKernelGGL(k_flash_f32<false>, grid, dim3(256), 0, ctx->stream, (const float*)q,
-                       q_rows, pos0, n_rows, ring.k, ring.v, ring.sp, ring.seq_stride, ring.C,
-                       ring.window, out, out_rows);
+    hipLaunchKernelGGL(ring.bf16 ? k_flash_x<true> : k_flash_x<false>,
+                       dim3((unsigned)((rows_max + QT - 1) / QT), nh, (unsigned)B), dim3(256), 0,
+                       ctx->stream, (const float*)q, q_rows, pos0, n_rows, ring.k, ring.v, ring.sp,
+                       ring.seq_stride, ring.C, ring.window, out, out_rows);
   MB_HIP(ctx, hipGetLastError());
   return MB_OK;
 }
