@@ -84,11 +84,15 @@ struct LayerW {
   // weight storage, bf16 and unscaled (the kernels apply gamma to the rows)
   const void *attn_wk, *fc_in_wk, *proj_wk, *fc_out_wk;
   const void *attn_wx, *fc_in_wx, *proj_wx, *fc_out_wx;  // null in fp32-KV contexts
+  // fp32-KV contexts: three-plane copies of the same four (launch_split_w3),
+  // made by the first prompt call that is large enough to read them
+  const void *attn_w3, *fc_in_w3, *proj_w3, *fc_out_w3;
 };
 
 // Every weight a model call needs, resolved from the uploaded tensors.
 struct ModelW {
   std::vector<LayerW> layers;
+  bool planes = false;  // the layers' three-plane copies are made
   const float *lnf_w, *lnf_b, *wte;
   AudioTables audio_emb;
   LayerW local;
@@ -289,7 +293,10 @@ int launch_append_attn(mb_ctx* ctx, const RingView& ring, int B, const void* qkv
                        const Rows& qo_rows, float* out, const Rows& out_rows, int pos_const = -1);
 int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                              const void* q, int q_dtype, const Rows& q_rows, const int32_t* pos0,
-                             const int32_t* n_rows, float* out, const Rows& out_rows);
+                             const int32_t* n_rows, float* out, const Rows& out_rows,
+                             int out_planes = 0);
+// (out_planes 2 or 3, fp32 queries: `out` is instead a planes operand of
+// 768-wide rows, the packed rows of out_rows.)
 // Chunks of up to 32 consecutive rows per sequence against long windows
 // (the codec's stages), out of the causal windowed rule: qkv holds the fused
 // fp32 rows (q | k | v, ring.heads x 64 each); every row is roped and written
@@ -364,6 +371,23 @@ int launch_split_w(mb_ctx* ctx, const float* Wt, int K, int N, void* Wx, bool ti
 int launch_gemm_x3(mb_ctx* ctx, int epi, const float* A, int64_t lda, const void* Wx, int N,
                    int K, const float* bias, float* Cm, int64_t ldc, int M, const float* lnc,
                    const float* lnd);
+
+// Prefill-sized projections on planes operands (gemm_planes.hip).  A planes
+// operand of M rows holds whole 16-row blocks of them, 2 `planes` bytes per
+// value.  launch_ln_planes writes the planes of (x - mean) rstd (times gamma
+// if not null) of 768-wide rows, and
+// launch_gemm_planes computes epi(A W + lnd + bias) from pa planes of A and pw
+// of W (2 x 2: the products of launch_gemm_x3, on its weight copies; 2 x 1:
+// launch_gemm_x2's; 3 x 3: fp32 products to 2^-24, on launch_split_w3's copies
+// of a column-block-major W, 6 K N bytes).  out_planes (GELU epilogues): the result goes there as
+// the planes of the next projection's operand, not to Cm.  N a multiple of
+// 128, K of 32.
+int launch_ln_planes(mb_ctx* ctx, int planes, const float* x, int64_t ldx, int M,
+                     const float* gamma, void* out);
+int launch_split_w3(mb_ctx* ctx, const float* Wt, int K, int N, void* Wx);
+int launch_gemm_planes(mb_ctx* ctx, int pa, int pw, int epi, const void* Ap, const void* Wx, int N,
+                       int K, const float* lnd, const float* bias, float* Cm, int64_t ldc, int M,
+                       void* out_planes = nullptr);
 
 // bf16 weight storage (mb_set_weight_storage).  launch_round_bf16: Wr =
 // bf16(W) kept as fp32 (round to nearest even), the weights every other copy

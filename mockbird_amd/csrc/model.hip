@@ -163,6 +163,7 @@ int resolve(mb_ctx* ctx, bool global, bool local) {
     m.audio_emb.t[k] = get("core.model.audio_embeddings." + std::to_string(k) + ".weight", {CODES, D});
   if (global) {
     m.layers.assign(ctx->cfg.n_layers, LayerW{});
+    m.planes = false;
     for (int l = 0; l < ctx->cfg.n_layers; l++)
       resolve_layer(ctx, "core.model.transformer.h." + std::to_string(l) + ".", m.layers[l], missing);
     m.lnf_w = get("core.model.transformer.ln_f.weight", {D});
@@ -205,22 +206,94 @@ struct Act {
   float *x, *norm, *qkv, *q, *att, *ffn, *logits;
 };
 
-int activations(mb_ctx* ctx, int64_t M, Act& a) {
+// (`planes`: what a prompt call on planes keeps in norm, att and ffn)
+int activations(mb_ctx* ctx, int64_t rows, Act& a, int planes = 0) {
+  const int64_t M = (rows + 15) / 16 * 16;  // whole 16-row blocks of planes
+  const size_t e = planes == 3 ? 6 : 4;
   a.x = (float*)scratch(ctx, "act_x", (size_t)M * D * 4);
-  a.norm = (float*)scratch(ctx, "act_norm", (size_t)M * D * 4);
+  a.norm = (float*)scratch(ctx, "act_norm", (size_t)M * D * e);
   a.qkv = (float*)scratch(ctx, "act_qkv", (size_t)M * QKV * 4);
   a.q = (float*)scratch(ctx, "act_q", (size_t)M * D * 4);
-  a.att = (float*)scratch(ctx, "act_att", (size_t)M * D * 4);
-  a.ffn = (float*)scratch(ctx, "act_ffn", (size_t)M * FFN * 4);
+  a.att = (float*)scratch(ctx, "act_att", (size_t)M * D * e);
+  a.ffn = (float*)scratch(ctx, "act_ffn", (size_t)M * FFN * e);
   a.logits = (float*)scratch(ctx, "act_logits", (size_t)M * CODES * 4);
   if (!a.x || !a.norm || !a.qkv || !a.q || !a.att || !a.ffn || !a.logits)
-    return fail(ctx, MB_ERR_NOMEM, "activation allocation failed (%lld rows)", (long long)M);
+    return fail(ctx, MB_ERR_NOMEM, "activation allocation failed (%lld rows)", (long long)rows);
   return MB_OK;
 }
 
 int cancelled(mb_ctx* ctx) {
   if (ctx->cancel.load()) return fail(ctx, MB_ERR_CANCELLED, "cancelled");
   return MB_OK;
+}
+
+// The planes that a prompt pass of M rows runs its projections on
+// (gemm_planes.hip): 2 in bf16-KV contexts, 3 in fp32-KV ones, 0 below the
+// sizes from which that is the faster way.  A whole 12-layer pass, other
+// kernels -> planes: bf16 K/V 2560 / 3200 / 5120 / 10240 rows 2581 -> 2625,
+// 3099 -> 2923, 4034 -> 3688, 7634 -> 6682 us; fp32 K/V 1280 / 1920 / 3200 /
+// 10240 rows 2858 -> 2887, 6080 -> 3466, 7841 -> 4342, 20472 -> 11078 us.
+constexpr int kPlanesMinRows2 = 2800, kPlanesMinRows3 = 1300;
+int prompt_planes(const mb_ctx* ctx, int64_t M) {
+  if (ctx->cfg.kv_dtype == MB_KV_BF16) return M >= kPlanesMinRows2 ? 2 : 0;
+  return M >= kPlanesMinRows3 ? 3 : 0;
+}
+
+// The three-plane weight copies of every global layer.
+int weight_planes(mb_ctx* ctx) {
+  ModelW& m = ctx->model;
+  if (m.planes) return MB_OK;
+  for (size_t l = 0; l < m.layers.size(); l++) {
+    LayerW& w = m.layers[l];
+    const std::string key = "#fold/h" + std::to_string(l);
+    auto one = [&](const char* name, const float* Wt, int K, int N, const void*& w3) {
+      float* p = internal_tensor(ctx, key + name, (int64_t)K * N * 3 / 2);  // 3 K N bf16
+      if (!p) return fail(ctx, MB_ERR_NOMEM, "weight planes allocation failed (%s)", key.c_str());
+      w3 = p;
+      return launch_split_w3(ctx, Wt, K, N, p);
+    };
+    int rc;
+    if ((rc = one(".attn.3", w.attn_wg, D, QKV, w.attn_w3)) ||
+        (rc = one(".proj.3", w.proj_wt, D, D, w.proj_w3)) ||
+        (rc = one(".fc_in.3", w.fc_in_wg, D, FFN, w.fc_in_w3)) ||
+        (rc = one(".fc_out.3", w.fc_out_wt, FFN, D, w.fc_out_w3)))
+      return rc;
+  }
+  m.planes = true;
+  return MB_OK;
+}
+
+// run_layer's prompt form on P planes: each operand's planes are written by
+// the kernel that computes its values.  The LayerNorms run apart (their rows
+// normalised once, not once per column tile) with gamma in the folded
+// weights; bf16 weights in bf16-KV contexts are unscaled and take it with the
+// rows.
+int run_layer_planes(mb_ctx* ctx, int P, const LayerW& w, const RingView& ring, int B, int rows_max,
+                     int M, const int32_t* pos0, const int32_t* n_rows, const int32_t* row_off, Act& a) {
+  const bool w1 = P == 2 && ctx->w_bf16;
+  const int pw = w1 ? 1 : P;
+  const void* attn = P == 3 ? w.attn_w3 : w.attn_wx;
+  const void* proj = P == 3 ? w.proj_w3 : w.proj_wx;
+  const void* fc_in = P == 3 ? w.fc_in_w3 : w.fc_in_wx;
+  const void* fc_out = P == 3 ? w.fc_out_w3 : w.fc_out_wx;
+  Rows qkv_rows, q_rows;
+  qkv_rows.row_stride = QKV;
+  q_rows.row_stride = D;
+  qkv_rows.row_off = q_rows.row_off = row_off;
+  int rc;
+  if ((rc = launch_ln_planes(ctx, P, a.x, D, M, w1 ? w.ln1_w : nullptr, a.norm)) ||
+      (rc = launch_gemm_planes(ctx, P, pw, EPI_STORE, a.norm, attn, QKV, D, w.attn_d, w.attn_b, a.qkv,
+                               QKV, M)) ||
+      (rc = launch_ring_write(ctx, ring, B, rows_max, a.qkv, MB_DT_F32, qkv_rows, pos0, n_rows, a.q,
+                              MB_DT_F32, q_rows)) ||
+      (rc = launch_prefill_attention(ctx, ring, B, rows_max, a.q, MB_DT_F32, q_rows, pos0, n_rows,
+                                     a.att, q_rows, P)) ||
+      (rc = launch_gemm_planes(ctx, P, pw, EPI_ADD, a.att, proj, D, D, nullptr, w.proj_b, a.x, D, M)) ||
+      (rc = launch_ln_planes(ctx, P, a.x, D, M, w1 ? w.ln2_w : nullptr, a.norm)) ||
+      (rc = launch_gemm_planes(ctx, P, pw, EPI_GELU, a.norm, fc_in, FFN, D, w.fc_in_d, w.fc_in_b,
+                               nullptr, 0, M, a.ffn)))
+    return rc;
+  return launch_gemm_planes(ctx, P, pw, EPI_ADD, a.ffn, fc_out, D, FFN, nullptr, w.fc_out_b, a.x, D, M);
 }
 
 // One d=768 layer over M rows held in a.x.  Rows belong to B sequences with
@@ -626,8 +699,13 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
     memcpy(packed.data() + (size_t)off[b] * ROW, ids + (size_t)b * rows_max * ROW,
            (size_t)n_rows[b] * ROW * 4);
   if ((rc = check_ids(ctx, packed.data(), M))) return rc;
+  int planes = prompt_planes(ctx, M);
+  if (planes == 3 && weight_planes(ctx)) {
+    planes = 0;  // no room for the copies: the kernels that need none
+    (void)hipGetLastError();
+  }
   Act a;
-  if ((rc = activations(ctx, M, a))) return rc;
+  if ((rc = activations(ctx, M, a, planes))) return rc;
   int32_t* d_ids = (int32_t*)scratch(ctx, "prefill_ids", (size_t)M * ROW * 4);
   int32_t* d_meta = (int32_t*)scratch(ctx, "prefill_meta", (size_t)B * 4 * 4);
   float* d_hidden = (float*)scratch(ctx, "hidden", (size_t)B * D * 4);
@@ -649,8 +727,10 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
   if ((rc = launch_embed_rows(ctx, d_ids, (int)M, m.wte, ctx->cfg.vocab, m.audio_emb, a.x))) return rc;
   for (int l = 0; l < layer_count; l++) {
     if ((rc = cancelled(ctx))) return rc;
-    if ((rc = run_layer(ctx, m.layers[l], global_ring(ctx, l), B, rows_max, M, d_pos0, d_n, d_off,
-                        true, ctx->cfg.capacity, a)))
+    if ((rc = planes ? run_layer_planes(ctx, planes, m.layers[l], global_ring(ctx, l), B, rows_max,
+                                        (int)M, d_pos0, d_n, d_off, a)
+                     : run_layer(ctx, m.layers[l], global_ring(ctx, l), B, rows_max, M, d_pos0, d_n,
+                                 d_off, true, ctx->cfg.capacity, a)))
       return rc;
   }
   if (last_hidden) {

@@ -18,11 +18,11 @@
 #include "kv_types.h"
 #include "lds_dma.h"
 #include "mb_internal.h"
+#include "planes.h"
 #include "rope.h"
 
 namespace mb {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -491,50 +491,6 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
 
 // ------------------------------------------------------------ fp32 queries
 
-// Three bf16 planes of a float: x = h + m + l exactly.  Cutting the low 16
-// bits leaves 8 significant bits, the remainder (exact) has at most 16, and
-// cutting that one leaves at most 8: three bf16 numbers.  (Overflow cannot
-// happen, as rounding to bf16 could; below 2^-110 the low plane may be
-// denormal.)  Eight values at a time, packed as MFMA operands.
-struct Planes {
-  bf16x8_t p[3];
-};
-__device__ __forceinline__ Planes split3(const float (&v)[8]) {
-  uint32_t w[3][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t a = __float_as_uint(v[2 * i]), b = __float_as_uint(v[2 * i + 1]);
-    w[0][i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
-    const float ra = v[2 * i] - __uint_as_float(a & 0xffff0000u);
-    const float rb = v[2 * i + 1] - __uint_as_float(b & 0xffff0000u);
-    const uint32_t ma = __float_as_uint(ra), mb = __float_as_uint(rb);
-    w[1][i] = __builtin_amdgcn_perm(mb, ma, 0x07060302u);
-    const float la = ra - __uint_as_float(ma & 0xffff0000u);
-    const float lb = rb - __uint_as_float(mb & 0xffff0000u);
-    w[2][i] = __builtin_amdgcn_perm(__float_as_uint(lb), __float_as_uint(la), 0x07060302u);
-  }
-  Planes r;
-#pragma unroll
-  for (int k = 0; k < 3; k++)
-    r.p[k] = __builtin_bit_cast(bf16x8_t, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
-  return r;
-}
-
-// f(i, j) for the plane pairs of a product of KP by three planes that are
-// kept, the smallest first: the planes' weights are 2^0, 2^-8, 2^-16, and
-// pairs beyond i + j = 2 are below 2^-24 of the product.
-template <int KP, class F>
-__device__ __forceinline__ void plane_pairs(F f) {
-  using std::integral_constant;
-  auto at = [&](auto i, auto j) {
-    if constexpr (decltype(i)::value < KP) f(i, j);
-  };
-  integral_constant<int, 0> c0;
-  integral_constant<int, 1> c1;
-  integral_constant<int, 2> c2;
-  at(c2, c0); at(c0, c2); at(c1, c1); at(c1, c0); at(c0, c1); at(c0, c0);
-}
-
 // Q fp32 [B][rows_max][768] (roped), K/V fp32 or bf16 ring, fp32 output: the
 // model's prompt passes.  Tile classes and online softmax are k_flash_bf16's;
 // every fp32 operand enters the bf16 matrix unit as three exact bf16 planes
@@ -557,7 +513,8 @@ __device__ __forceinline__ void plane_pairs(F f) {
 // registers), two waves per workgroup (20.3 / 96.3 / 121.1 us, fp32), and
 // k_flash_bf16's snake order (equal).  With the fp32 MFMA kernel the same
 // calls took 28.3 / 109.3 / 130.6 us (fp32) and 29.1 / 106.2 / 121.7 (bf16).
-template <bool KV_BF16>
+// PO: the planes of the output (the O projection's operand) instead of fp32.
+template <bool KV_BF16, int PO>
 __global__ __launch_bounds__(256, 3) void k_flash_x(
     const float* __restrict__ q, Rows q_rows, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ n_rows, const void* __restrict__ ring_k,
@@ -681,7 +638,7 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
 #pragma unroll
         for (int p = 0; p < KP; p++)
           ka[sb][p] = *(const bf16x8_t*)&Ks[bb][p][swz(sb * 16 + qcol, kc * 4 + grp)];
-      plane_pairs<KP>([&](auto i, auto j) {
+      plane_products<KP, 3>([&](auto i, auto j) {
 #pragma unroll
         for (int sb = 0; sb < SB; sb++)
           s[sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[sb][i], qp[kc].p[j], s[sb], 0, 0, 0);
@@ -737,7 +694,7 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
           const bf16x4_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t*)&Vs[bb][p][e1]);
           va[d][p] = bf16x8_t{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
         }
-      plane_pairs<KP>([&](auto i, auto j) {
+      plane_products<KP, 3>([&](auto i, auto j) {
 #pragma unroll
         for (int d = 0; d < 4; d++)
           acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[d][i], pp.p[j], acc[d], 0, 0, 0);
@@ -762,9 +719,23 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
   const float l = col_sum(lsum);
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (r >= n) return;
-  float* op = out + row_at(out_rows, b, r) + h * HD;
+  if constexpr (PO == 0) {
+    float* op = out + row_at(out_rows, b, r) + h * HD;
 #pragma unroll
-  for (int d = 0; d < 4; d++) *(f32x4_t*)(op + d * 16 + grp * 4) = acc[d] * inv;
+    for (int d = 0; d < 4; d++) *(f32x4_t*)(op + d * 16 + grp * 4) = acc[d] * inv;
+  } else {
+    const int64_t row = (int64_t)out_rows.row_off[b] + r;
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+      const f32x4_t v = acc[d] * inv;
+      uint2 o[PO];
+      split4<PO>(make_float4(v[0], v[1], v[2], v[3]), o);
+#pragma unroll
+      for (int p = 0; p < PO; p++)
+        ((uint2*)out)[2 * plane_chunk(row, h * (HD / 8) + 2 * d + (grp >> 1), D / 32, PO, p) + (grp & 1)] =
+            o[p];
+    }
+  }
 }
 
 // ------------------------------------------------ short chunks, long windows
@@ -1248,7 +1219,10 @@ int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_m
 
 int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                              const void* q, int q_dtype, const Rows& q_rows, const int32_t* pos0,
-                             const int32_t* n_rows, float* out, const Rows& out_rows) {
+                             const int32_t* n_rows, float* out, const Rows& out_rows,
+                             int out_planes) {
+  if (out_planes && (q_dtype != MB_DT_F32 || !out_rows.row_off || ring.heads != H || out_planes != (ring.bf16 ? 2 : 3)))
+    return fail(ctx, MB_ERR_ARG, "attention planes: packed fp32 rows of the model's ring");
   if (q_dtype == MB_DT_BF16 && !ring.bf16)
     return fail(ctx, MB_ERR_ARG, "bf16 queries need a bf16 ring (the bf16 MFMA path)");
   if (B > 65535) return fail(ctx, MB_ERR_ARG, "at most 65535 sequences per prefill call");
@@ -1264,7 +1238,8 @@ int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_
                        ring.seq_stride, ring.C, ring.window, out, out_rows, ctx->xcds,
                        ctx->cus_per_xcd);
   else
-    hipLaunchKernelGGL(ring.bf16 ? k_flash_x<true> : k_flash_x<false>,
+    hipLaunchKernelGGL(ring.bf16 ? (out_planes ? k_flash_x<true, 2> : k_flash_x<true, 0>)
+                                 : (out_planes ? k_flash_x<false, 3> : k_flash_x<false, 0>),
                        dim3((unsigned)((rows_max + QT - 1) / QT), nh, (unsigned)B), dim3(256), 0,
                        ctx->stream, (const float*)q, q_rows, pos0, n_rows, ring.k, ring.v, ring.sp,
                        ring.seq_stride, ring.C, ring.window, out, out_rows);

@@ -598,3 +598,46 @@ def test_device_frame_loop_stops_voices():
     assert np.array_equal(h.cpu().numpy()[going], want_h[going])
     # the latch: once 0, a voice's flag stays 0
     assert (np.diff(got_cont, axis=0) <= 0).all()
+
+
+@pytest.mark.parametrize("kv,weights,voices", [
+    (mb.MB_KV_F32, mb.MB_W_F32, 7), (mb.MB_KV_F32, mb.MB_W_BF16, 7),
+    (mb.MB_KV_BF16, mb.MB_W_F32, 14), (mb.MB_KV_BF16, mb.MB_W_BF16, 14)])
+def test_large_prompt_batches_equal_single_prompts(kv, weights, voices):
+    """A batch whose rows pass the sizes from which prompts run on planes
+    operands (1300 rows fp32 K/V, 2800 bf16; the total no multiple of 16 or
+    64, one voice of a single row) gives every voice's hidden rows and ring as
+    its own small call does, within what the two kernels' roundings give:
+    fp32 sums in another order through 2 layers (1e-5), split-bf16 products
+    and bf16 K/V (within 2^-16 of the product, K/V steps of 2^-9: 5e-3)."""
+    say(f"large prompt batch kv={kv} weights={weights}")
+    L, V = 2, 64
+    w = synth.model_weights(n_layers=L, vocab=V, seed=5, bias_std=0.02, ln_std=0.1)
+    g = np.random.default_rng(6)
+    n = g.integers(200, 231, size=voices).astype(np.int32)
+    n[1] = 1
+    n[0] += 1 - (int(n.sum()) & 1)  # an odd total
+    R = int(n.max())
+    ids = np.full((voices, R, 17), 1024, np.int32)
+    ids[:, :, 0] = g.integers(0, V, size=(voices, R))
+    ids[:, 3:90, 1:] = g.integers(0, 1024, size=(voices, 87, 16))
+    assert int(n.sum()) >= (1300 if kv == mb.MB_KV_F32 else 2800) and n.sum() % 16
+    tol = 1e-5 if kv == mb.MB_KV_F32 else 5e-3
+    with _ctx(w, L, V, voices, 256, kv) as ctx, _ctx(w, L, V, 1, 256, kv) as one:
+        for c in (ctx, one):
+            c.set_weight_storage(weights)
+        h = ctx.prefill_rows(ids, n)
+        last = ctx.prefill(ids, n)
+        worst = 0.0
+        for b in range(voices):
+            want = one.prefill_rows(ids[b:b + 1], n[b:b + 1])[0, :n[b]]
+            worst = max(worst, float(np.abs(h[b, :n[b]] - want).max()))
+            assert np.array_equal(last[b], h[b, n[b] - 1])
+            for l in range(L):
+                k, v, sp = ctx.read_ring(l, b)
+                k1, v1, sp1 = one.read_ring(l, 0)
+                assert np.array_equal(sp, sp1)
+                live = sp >= 0
+                assert np.abs(k - k1)[live].max() < 10 * tol and np.abs(v - v1)[live].max() < 10 * tol
+        say(f"  max difference {worst:.2e}")
+        assert worst < tol
