@@ -21,15 +21,12 @@
 #include "lds_dma.h"
 #include "mb_internal.h"
 #include "pick.h"
+#include "planes.h"
 
 namespace mb {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
 typedef float f32x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 // v = hi + lo in bf16 halves: hi = bf16(v), lo = bf16(v - hi), both rounded
 // to nearest even.  The high halves are converted in pairs and their fp32
@@ -425,7 +422,14 @@ __device__ __forceinline__ void stream_finish(f32x4_t (&acc)[MI][4], float (&sx)
 // It accumulates them from the A values it streams anyway -- sums of
 // x - x0 and (x - x0)^2 with x0 = x[row][0], so the variance does not cancel
 // -- which requires the workgroup to see the whole row (S == 1, K == 768).
-template <int MT, int ST, int EPI, bool LNF, bool TILED>
+//
+// PLANES: the products on the bf16 matrix unit.  A wave splits the A rows and
+// W columns it holds into three exact bf16 planes each (planes.h) and sums the
+// six plane products above 2^-24 in fp32: per 16 x 16 x 32 block 6 MFMAs of 16
+// cycles in place of 8 of 32.  Its error against float64 is the smaller one
+// (768-deep 2.5e-7 -> 2.1e-7, 3072-deep 5.0e-7 -> 4.3e-7 relative: fewer
+// roundings of the running sum).  stream_planes says where it is taken.
+template <int MT, int ST, int EPI, bool LNF, bool TILED, bool PLANES>
 __global__ __launch_bounds__(256) void k_gemm_stream(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ W, int N, int kw,
     const float* __restrict__ bias, float* __restrict__ Cm, int64_t ldc, int M,
@@ -438,77 +442,103 @@ __global__ __launch_bounds__(256) void k_gemm_stream(
   const int S = gridDim.z, split = blockIdx.z;
 
   f32x4_t acc[MI][4];
-#pragma unroll
-  for (int i = 0; i < MI; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float x0[MI], sx[MI], sxx[MI];
-
-  {
-    // Rows past M read row M - 1 (in bounds, no branch); their sums are
-    // never stored.
-    const float* Ap[MI];
+  // Rows past M read row M - 1 (in bounds, no branch); their sums are
+  // never stored.
+  const float* Ap[MI];
 #pragma unroll
-    for (int i = 0; i < MI; i++) Ap[i] = A + (int64_t)min(m0 + 16 * i + l16, M - 1) * lda + 4 * r;
-    if (LNF) {
+  for (int i = 0; i < MI; i++) Ap[i] = A + (int64_t)min(m0 + 16 * i + l16, M - 1) * lda + 4 * r;
+  // TILED: W column-block-major, [N / 64][K][64] (launch_tile_w), so a
+  // workgroup streams one contiguous strip instead of 256 bytes of every row
+  const int64_t wstride = TILED ? 64 : N;
+  const float* Wp = TILED ? W + (int64_t)blockIdx.x * 64 * (4 * S * kw) + 4 * r * 64 + 4 * l16
+                          : W + (int64_t)4 * r * N + n;
+  // The wave's k range, in steps of CD 16-deep chunks: one on the fp32 matrix
+  // unit, or (`planes_`) two on the bf16 one.  A lane holds the same k values
+  // of A and W whichever they are (4r + t of each chunk), and any order of k
+  // will do, so the two forms load alike.
+  auto stream = [&](auto planes_) {
+    constexpr bool PL = decltype(planes_)::value;
+    constexpr int CD = PL ? 2 : 1, STEP = CD * kStreamChunk;
 #pragma unroll
-      for (int i = 0; i < MI; i++) {
+    for (int i = 0; i < MI; i++) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (LNF) {
         x0[i] = Ap[i][-4 * r];
         sx[i] = 0.f;
         sxx[i] = 0.f;
       }
     }
-    // TILED: W column-block-major, [N / 64][K][64] (launch_tile_w), so a
-    // workgroup streams one contiguous strip instead of 256 bytes of every row
-    const int64_t wstride = TILED ? 64 : N;
-    const float* Wp = TILED ? W + (int64_t)blockIdx.x * 64 * (4 * S * kw) + 4 * r * 64 + 4 * l16
-                            : W + (int64_t)4 * r * N + n;
-    float4 a[ST][MI], w[ST][4];
+    f32x4_t a[ST][MI][CD], w[ST][4 * CD];
     auto load = [&](int st, int k) {
 #pragma unroll
-      for (int t = 0; t < 4; t++) w[st][t] = *(const float4*)(Wp + (int64_t)(k + t) * wstride);
+      for (int t = 0; t < 4 * CD; t++)
+        w[st][t] = *(const f32x4_t*)(Wp + (int64_t)(k + (t >> 2) * kStreamChunk + (t & 3)) * wstride);
 #pragma unroll
-      for (int i = 0; i < MI; i++) a[st][i] = *(const float4*)(Ap[i] + k);
+      for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int c = 0; c < CD; c++) a[st][i][c] = *(const f32x4_t*)(Ap[i] + k + c * kStreamChunk);
     };
     auto mma = [&](int st) {
       if (LNF) {
 #pragma unroll
-        for (int i = 0; i < MI; i++) {
-          const float e0 = a[st][i].x - x0[i], e1 = a[st][i].y - x0[i];
-          const float e2 = a[st][i].z - x0[i], e3 = a[st][i].w - x0[i];
-          sx[i] += (e0 + e1) + (e2 + e3);
-          sxx[i] = fmaf(e0, e0, fmaf(e1, e1, fmaf(e2, e2, fmaf(e3, e3, sxx[i]))));
-        }
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+          for (int c = 0; c < CD; c++) {
+            const float e0 = a[st][i][c][0] - x0[i], e1 = a[st][i][c][1] - x0[i];
+            const float e2 = a[st][i][c][2] - x0[i], e3 = a[st][i][c][3] - x0[i];
+            sx[i] += (e0 + e1) + (e2 + e3);
+            sxx[i] = fmaf(e0, e0, fmaf(e1, e1, fmaf(e2, e2, fmaf(e3, e3, sxx[i]))));
+          }
       }
-#pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const float4 wt = w[st][t];
+      if constexpr (PL) {
+        Planes ap[MI];
 #pragma unroll
         for (int i = 0; i < MI; i++) {
-          const float av = t == 0 ? a[st][i].x : t == 1 ? a[st][i].y : t == 2 ? a[st][i].z : a[st][i].w;
-          acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wt.x, acc[i][0], 0, 0, 0);
-          acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wt.y, acc[i][1], 0, 0, 0);
-          acc[i][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wt.z, acc[i][2], 0, 0, 0);
-          acc[i][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, wt.w, acc[i][3], 0, 0, 0);
+          float v[8];
+#pragma unroll
+          for (int e = 0; e < 8; e++) v[e] = a[st][i][e >> 2][e & 3];
+          ap[i] = split3(v);
         }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          float v[8];
+#pragma unroll
+          for (int t = 0; t < 8; t++) v[t] = w[st][t][j];
+          const Planes wp = split3(v);
+          plane_products<3, 3>([&](auto pa, auto pw) {
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ap[i].p[pa], wp.p[pw], acc[i][j], 0, 0, 0);
+          });
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+          for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st][i][0][t], w[st][t][j], acc[i][j], 0, 0, 0);
       }
     };
-    // Prefetch ST - 1 chunks, then per chunk: issue the load ST - 1 ahead and
-    // run the MFMAs of the oldest stage.  Past the end the last chunk is
+    // Prefetch ST - 1 steps, then per step: issue the load ST - 1 ahead and
+    // run the MFMAs of the oldest stage.  Past the end the last step is
     // re-read (in bounds, unused), so the loop body has no load branch and
     // each stage's MFMAs wait only for that stage's loads.  The main loop
-    // runs whole groups of ST chunks with no branch inside: a stage skipped
+    // runs whole groups of ST steps with no branch inside: a stage skipped
     // on some path would leave its load pending at the loop header, and the
     // compiler then drains every load in flight there (vmcnt(0)) on every
-    // iteration.  The nc mod ST chunks left over (already in flight) follow.
-    const int k0 = (split * 4 + wave) * kw, k1 = k0 + kw, nc = kw / kStreamChunk;
+    // iteration.  The nc mod ST steps left over (already in flight) follow.
+    const int k0 = (split * 4 + wave) * kw, k1 = k0 + kw, nc = kw / STEP;
 #pragma unroll
-    for (int s = 0; s < ST - 1; s++) load(s, min(k0 + s * kStreamChunk, k1 - kStreamChunk));
+    for (int s = 0; s < ST - 1; s++) load(s, min(k0 + s * STEP, k1 - STEP));
     int c = 0;
     for (; c + ST <= nc; c += ST) {
 #pragma unroll
       for (int s = 0; s < ST; s++) {
-        load((s + ST - 1) % ST, min(k0 + (c + s + ST - 1) * kStreamChunk, k1 - kStreamChunk));
+        load((s + ST - 1) % ST, min(k0 + (c + s + ST - 1) * STEP, k1 - STEP));
         __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the MFMAs
         mma(s);
       }
@@ -516,6 +546,20 @@ __global__ __launch_bounds__(256) void k_gemm_stream(
 #pragma unroll
     for (int s = 0; s < ST - 1; s++)
       if (c + s < nc) mma(s);
+  };
+  if constexpr (PLANES) {
+    stream(std::true_type{});
+    // An infinite operand has no planes (inf - inf) and its products come out
+    // NaN; a wave that sees one takes its range again in fp32, so infinities
+    // and NaN reach the output as fp32 products give them.
+    float nan = 0.f;
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) nan += (acc[i][j][0] + acc[i][j][1]) + (acc[i][j][2] + acc[i][j][3]);
+    if (__ballot(!(fabsf(nan) < INFINITY))) stream(std::false_type{});
+  } else {
+    stream(std::false_type{});
   }
 
   stream_finish<MI, EPI, LNF>(acc, sx, sxx, x0, 4 * S * kw, bias, Cm, ldc, M, N, part, lnc, lnd);
@@ -734,6 +778,18 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ p
   *(float4*)cp = epilogue4<EPI>(sum, bias, col, cp);
 }
 
+// Whether a streaming launch multiplies bf16 planes (k_gemm_stream's PLANES):
+// 48- and 64-row tiles, and 32-row tiles over at least 512 k.  There the fp32
+// matrix rate bounds the loop; smaller tiles wait for W, and the splits only
+// add to that.  fp32 MFMA -> planes, us: 2304 x 768 at 281 / 500 / 1000 rows
+// 12.3 -> 10.7, 34.4 -> 24.7, 57.7 -> 36.8 (48- and 64-row tiles); 768 x 3072
+// at 100 / 281 / 1000 rows 11.3 -> 10.9, 17.5 -> 15.8, 39.6 -> 31.5 (32-row
+// ones); 256 x 256 at 2048 rows 4.9 -> 5.2, 768 x 768 at 64 rows 5.5 -> 6.1
+// (16-row tiles).
+static bool stream_planes(int mt, int K, int kw) {
+  return kw % (2 * kStreamChunk) == 0 && (mt >= 48 || (mt == 32 && K >= 512));
+}
+
 // part_ext (optional, part_cap floats) holds the split-K partials instead of
 // the context's growable scratch.
 template <int MT, int ST, bool LNF>
@@ -757,6 +813,7 @@ static int stream_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, cons
   }
   dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)S);
   const int kw = K / (4 * S);
+  const bool planes = stream_planes(MT, K, kw);
   if (LNF && epi != EPI_STORE && epi != EPI_GELU && epi != EPI_GELU_ERF)
     return fail(ctx, MB_ERR_ARG, "folded LayerNorm gemm has no epilogue %d", epi);
   with_epi(epi, [&](auto e) {
@@ -764,14 +821,20 @@ static int stream_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, cons
     // folded weights (LNF) always come tiled from launch_fold_ln
     if constexpr (LNF) {
       if constexpr (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF)
-        hipLaunchKernelGGL((k_gemm_stream<MT, ST, E, true, true>), grid, dim3(256), 0, ctx->stream,
-                           A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc, lnd);
+        hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, true, true, (MT > 16)>
+                                   : k_gemm_stream<MT, ST, E, true, true, false>),
+                           grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part,
+                           lnc, lnd);
     } else if (tiled) {
-      hipLaunchKernelGGL((k_gemm_stream<MT, ST, E, false, true>), grid, dim3(256), 0, ctx->stream,
-                         A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc, lnd);
+      hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, false, true, (MT > 16)>
+                                 : k_gemm_stream<MT, ST, E, false, true, false>),
+                         grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc,
+                         lnd);
     } else {
-      hipLaunchKernelGGL((k_gemm_stream<MT, ST, E, false, false>), grid, dim3(256), 0, ctx->stream,
-                         A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc, lnd);
+      hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, false, false, (MT > 16)>
+                                 : k_gemm_stream<MT, ST, E, false, false, false>),
+                         grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc,
+                         lnd);
     }
   });
   if (S > 1) {

@@ -62,6 +62,65 @@ def test_linear_matches_oracle(ctx, M, N, K):
         assert err < 1e-4, (epi, err)
 
 
+PLANE_SHAPES = [  # (M, N, K): 32-, 48- and 64-row tiles of the streaming kernel on planes
+    (100, 768, 3072), (193, 2304, 768), (240, 2304, 768), (281, 3072, 768), (1023, 2304, 768),
+    (2049, 768, 256), (600, 768, 512), (999, 768, 3072),
+]
+
+
+@pytest.mark.parametrize("M,N,K", PLANE_SHAPES)
+def test_linear_planes_hold_fp32(ctx, M, N, K):
+    """Products of three bf16 planes stand for fp32 ones: each is within
+    3 2^-24 of |a w| (the plane pairs left out) and the fp32 sums round at
+    most K / 128 times per wave beyond that, so an output is within
+    8 2^-24 sum |a w| of float64 -- operands over 30 binary orders, where a
+    two-plane split is off by 2^-16."""
+    torch = pytest.importorskip("torch")
+    say(f"linear planes M={M} N={N} K={K}")
+    g = np.random.default_rng([M, N, K, 1])
+    A = (g.standard_normal((M, K)) * 2.0 ** g.integers(-15, 15, size=(M, K))).astype(np.float32)
+    W = (g.standard_normal((K, N)) * 0.02).astype(np.float32)
+    dev = torch.device("cuda")
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    tA, tW = torch.from_numpy(A).to(dev), torch.from_numpy(W).to(dev)
+    tC = torch.zeros((M, N), device=dev)
+    ctx.linear_dev(M, N, K, tA.data_ptr(), K, tW.data_ptr(), None, tC.data_ptr(), N)
+    torch.cuda.synchronize()
+    want = tA.double() @ tW.double()
+    size = tA.double().abs() @ tW.double().abs()
+    worst = float(((tC.double() - want).abs() / size).max()) * 2 ** 24
+    say(f"  worst error {worst:.2f} x 2^-24 sum |a w|")
+    assert worst < 8
+
+
+def test_linear_planes_keep_infinities_and_nan(ctx):
+    """An infinity has no planes: the tile that holds one is taken in fp32, so
+    infinities, their NaN sums and the finite rows beside them are what fp32
+    products give."""
+    torch = pytest.importorskip("torch")
+    say("linear planes: infinities")
+    M, N, K = 281, 2304, 768
+    g = np.random.default_rng(77)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    W = np.abs(g.standard_normal((K, N), dtype=np.float32)) * np.float32(0.02) + np.float32(1e-3)
+    A[5, 3], A[70, 700], A[200, 10], A[200, 400], A[280, 767] = np.inf, -np.inf, np.inf, -np.inf, np.nan
+    W[100, 9] = np.inf
+    A[:, 100] = np.where(A[:, 100] == 0, 1, A[:, 100])
+    A[30, 100] = 3.0e38
+    dev = torch.device("cuda")
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    tA, tW = torch.from_numpy(A).to(dev), torch.from_numpy(W).to(dev)
+    tC = torch.zeros((M, N), device=dev)
+    ctx.linear_dev(M, N, K, tA.data_ptr(), K, tW.data_ptr(), None, tC.data_ptr(), N)
+    torch.cuda.synchronize()
+    want = (tA.double() @ tW.double()).float().cpu().numpy()
+    got = tC.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    assert np.abs(got[fin] - want[fin]).max() <= 1e-4 * np.abs(want[fin]).max()
+
+
 def test_linear_is_deterministic_and_strided(ctx):
     """Split-K partials are summed in split order by whichever block finishes
     last, so repeated calls are bit-identical; A and C may be row-strided."""
