@@ -309,6 +309,8 @@ int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_m
                             const int32_t* n_rows, float* out, const Rows& out_rows,
                             float* part = nullptr);
 int launch_fill_i32(mb_ctx* ctx, int32_t* p, int64_t n, int32_t value);
+// the first n words of `rows` rows, `stride` words apart
+int launch_fill_rows_i32(mb_ctx* ctx, int32_t* p, int rows, int64_t stride, int64_t n, int32_t value);
 int launch_fill_kv(mb_ctx* ctx, void* p, int64_t n, float value);
 
 // gemm.hip.  EPI_SCALE_ADD (the codec's layer scale) reads the `bias`

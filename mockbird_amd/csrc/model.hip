@@ -682,7 +682,6 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
   if (rows_max < 1 || rows_max > ctx->cfg.max_rows)
     return fail(ctx, MB_ERR_ARG, "rows_max %d out of [1, %d]", rows_max, ctx->cfg.max_rows);
   if ((rc = need_model(ctx))) return rc;
-  std::vector<int32_t> off(B), last(B), zeros(B, 0);
   int64_t M = 0;
   for (int b = 0; b < B; b++) {
     if (n_rows[b] < 1 || n_rows[b] > rows_max)
@@ -690,15 +689,21 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
     if (n_rows[b] > ctx->cfg.capacity)
       return fail(ctx, MB_ERR_RANGE, "prompt of %d rows exceeds the KV ring (%d slots)", n_rows[b],
                   ctx->cfg.capacity);
-    off[b] = (int32_t)M;
     M += n_rows[b];
-    last[b] = (int32_t)(M - 1);
   }
-  std::vector<int32_t> packed((size_t)M * ROW);
-  for (int b = 0; b < B; b++)
-    memcpy(packed.data() + (size_t)off[b] * ROW, ids + (size_t)b * rows_max * ROW,
-           (size_t)n_rows[b] * ROW * 4);
-  if ((rc = check_ids(ctx, packed.data(), M))) return rc;
+  // what the device reads, in one block (one copy): per sequence its first
+  // row, rows, position and last row, then the packed rows' ids
+  std::vector<int32_t> meta((size_t)4 * B + (size_t)M * ROW);
+  int32_t *const off = meta.data(), *const packed = meta.data() + 4 * B;
+  for (int64_t b = 0, row = 0; b < B; b++) {
+    off[b] = (int32_t)row;
+    off[B + b] = n_rows[b];
+    off[2 * B + b] = 0;
+    memcpy(packed + row * ROW, ids + (size_t)b * rows_max * ROW, (size_t)n_rows[b] * ROW * 4);
+    row += n_rows[b];
+    off[3 * B + b] = (int32_t)(row - 1);
+  }
+  if ((rc = check_ids(ctx, packed, M))) return rc;
   int planes = prompt_planes(ctx, M);
   if (planes == 3 && weight_planes(ctx)) {
     planes = 0;  // no room for the copies: the kernels that need none
@@ -706,23 +711,20 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
   }
   Act a;
   if ((rc = activations(ctx, M, a, planes))) return rc;
-  int32_t* d_ids = (int32_t*)scratch(ctx, "prefill_ids", (size_t)M * ROW * 4);
-  int32_t* d_meta = (int32_t*)scratch(ctx, "prefill_meta", (size_t)B * 4 * 4);
+  int32_t* d_meta = (int32_t*)scratch(ctx, "prefill_meta", meta.size() * 4);
   float* d_hidden = (float*)scratch(ctx, "hidden", (size_t)B * D * 4);
-  if (!d_ids || !d_meta || !d_hidden) return fail(ctx, MB_ERR_NOMEM, "staging allocation failed");
+  if (!d_meta || !d_hidden) return fail(ctx, MB_ERR_NOMEM, "staging allocation failed");
   int32_t* d_off = d_meta;
   int32_t* d_n = d_meta + B;
   int32_t* d_pos0 = d_meta + 2 * B;
   int32_t* d_last = d_meta + 3 * B;
-  MB_HIP(ctx, hipMemcpyAsync(d_ids, packed.data(), (size_t)M * ROW * 4, hipMemcpyHostToDevice, ctx->stream));
-  MB_HIP(ctx, hipMemcpyAsync(d_off, off.data(), (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
-  MB_HIP(ctx, hipMemcpyAsync(d_n, n_rows, (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
-  MB_HIP(ctx, hipMemcpyAsync(d_pos0, zeros.data(), (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
-  MB_HIP(ctx, hipMemcpyAsync(d_last, last.data(), (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
+  int32_t* d_ids = d_meta + 4 * B;
+  MB_HIP(ctx, hipMemcpyAsync(d_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, ctx->stream));
   // a fresh utterance per sequence: every slot of its rings forgets its position
-  for (int l = 0; l < ctx->cfg.n_layers; l++)
-    if ((rc = launch_fill_i32(ctx, ctx->slot_pos + slot_base(ctx, l, 0), (int64_t)B * ctx->cfg.capacity, -1)))
-      return rc;
+  if ((rc = launch_fill_rows_i32(ctx, ctx->slot_pos, ctx->cfg.n_layers,
+                                 (int64_t)ctx->cfg.max_seqs * ctx->cfg.capacity,
+                                 (int64_t)B * ctx->cfg.capacity, -1)))
+    return rc;
   const ModelW& m = ctx->model;
   if ((rc = launch_embed_rows(ctx, d_ids, (int)M, m.wte, ctx->cfg.vocab, m.audio_emb, a.x))) return rc;
   for (int l = 0; l < layer_count; l++) {
@@ -738,20 +740,23 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
     MB_HIP(ctx, hipMemcpyAsync(last_hidden, d_hidden, (size_t)B * D * 4, hipMemcpyDeviceToHost,
                                ctx->stream));
   }
-  std::vector<float> rows;
   if (all_hidden) {
+    // straight to the caller's rows, one copy per run of full sequences
     if ((rc = launch_layernorm(ctx, a.x, D, nullptr, (int)M, m.lnf_w, m.lnf_b, a.norm, D))) return rc;
-    rows.resize((size_t)M * D);
-    MB_HIP(ctx, hipMemcpyAsync(rows.data(), a.norm, rows.size() * 4, hipMemcpyDeviceToHost,
-                               ctx->stream));
+    for (int b = 0; b < B;) {
+      int e = b + 1;
+      while (e < B && n_rows[e - 1] == rows_max) e++;
+      const int64_t rows = off[3 * B + e - 1] + 1 - off[b];
+      MB_HIP(ctx, hipMemcpyAsync(all_hidden + (size_t)b * rows_max * D, a.norm + (size_t)off[b] * D,
+                                 (size_t)rows * D * 4, hipMemcpyDeviceToHost, ctx->stream));
+      b = e;
+    }
   }
   MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (all_hidden) {
-    memset(all_hidden, 0, (size_t)B * rows_max * D * 4);
+  if (all_hidden)
     for (int b = 0; b < B; b++)
-      memcpy(all_hidden + (size_t)b * rows_max * D, rows.data() + (size_t)off[b] * D,
-             (size_t)n_rows[b] * D * 4);
-  }
+      memset(all_hidden + ((size_t)b * rows_max + n_rows[b]) * D, 0,
+             (size_t)(rows_max - n_rows[b]) * D * 4);
   return MB_OK;
 }
 

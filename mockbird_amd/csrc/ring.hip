@@ -16,7 +16,9 @@ namespace mb {
 
 // ------------------------------------------------------------------ fills
 
-__global__ void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t value) {
+// (row blockIdx.y, `stride` words apart)
+__global__ void k_fill_i32(int32_t* __restrict__ p, int64_t stride, int64_t n, int32_t value) {
+  p += blockIdx.y * stride;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     p[i] = value;
@@ -41,7 +43,14 @@ static int grid_for(int64_t n, int block) {
 
 int launch_fill_i32(mb_ctx* ctx, int32_t* p, int64_t n, int32_t value) {
   if (n <= 0) return MB_OK;
-  hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n, 256)), dim3(256), 0, ctx->stream, p, n, value);
+  return launch_fill_rows_i32(ctx, p, 1, 0, n, value);
+}
+
+int launch_fill_rows_i32(mb_ctx* ctx, int32_t* p, int rows, int64_t stride, int64_t n, int32_t value) {
+  if (n <= 0 || rows <= 0) return MB_OK;
+  for (int r0 = 0; r0 < rows; r0 += 65535)
+    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n, 256), (unsigned)std::min(rows - r0, 65535)),
+                       dim3(256), 0, ctx->stream, p + r0 * stride, stride, n, value);
   MB_HIP(ctx, hipGetLastError());
   return MB_OK;
 }
