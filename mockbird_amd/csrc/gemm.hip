@@ -16,6 +16,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "coherent.h"
 #include "gemm_epi.h"
 #include "kv_types.h"
 #include "lds_dma.h"
@@ -221,19 +222,6 @@ __device__ __forceinline__ float4 epilogue_regs(float4 v, float4 b, bool has_bia
     v.x = c.x + v.x; v.y = c.y + v.y; v.z = c.z + v.z; v.w = c.w + v.w;
   }
   return v;
-}
-
-// Two floats stored, and four loaded, as device-coherent accesses
-// (agent-scope relaxed atomics: sc1 stores and loads on gfx950).
-__device__ __forceinline__ void store_coherent(float* p, float a, float b) {
-  const uint64_t v = (uint64_t)__float_as_uint(a) | ((uint64_t)__float_as_uint(b) << 32);
-  __hip_atomic_store((uint64_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float4 load_coherent(const float* p) {
-  const uint64_t lo = __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t hi = __hip_atomic_load((const uint64_t*)p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return make_float4(__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)),
-                     __uint_as_float((uint32_t)hi), __uint_as_float((uint32_t)(hi >> 32)));
 }
 
 // The end of a streaming tile, shared by k_gemm_stream and k_gemm_x3: the

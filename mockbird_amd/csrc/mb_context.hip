@@ -79,6 +79,25 @@ int hip_fail(mb_ctx* ctx, hipError_t e, const char* what) {
   return fail(ctx, MB_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
+// The context's AttnSplit for a call on its stream: none while that stream is
+// captured (a replay would share it with later calls) or another stream's
+// calls may still be using it.
+static AttnSplit claim_split(mb_ctx* ctx) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (ctx->split_claimed && ctx->split_stream != ctx->stream) return {};
+  if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return {};
+  }
+  ctx->split_claimed = true;
+  ctx->split_stream = ctx->stream;
+  return {ctx->split_part, ctx->split_count};
+}
+// After the context's stream has been synchronised.
+static void release_split(mb_ctx* ctx) {
+  if (ctx->split_stream == ctx->stream) ctx->split_claimed = false;
+}
+
 void* scratch(mb_ctx* ctx, const char* name, size_t bytes) {
   Scratch& s = ctx->scratch[name];
   if (s.bytes >= bytes && s.ptr) return s.ptr;
@@ -220,7 +239,13 @@ int mb_create(const mb_config* cfg, mb_ctx** out) {
       e = hipMemcpy(ctx->rope_tab, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
       if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMemcpy(rope table)"); break; }
     }
-    ctx->device_bytes = 2 * (int64_t)ctx->ring_bytes + slots * 4 + (int64_t)kRopeTab * 32 * 8;
+    e = hipMalloc(&ctx->split_part, kSplitFloats * 4 + kSplitMaxUnits * 4);
+    if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMalloc(attention split)"); break; }
+    ctx->split_count = (int32_t*)(ctx->split_part + kSplitFloats);
+    rc = launch_fill_i32(ctx, ctx->split_count, kSplitMaxUnits, 0);
+    if (rc) break;
+    ctx->device_bytes = 2 * (int64_t)ctx->ring_bytes + slots * 4 + (int64_t)kRopeTab * 32 * 8 +
+                        (int64_t)(kSplitFloats + kSplitMaxUnits) * 4;
     // every slot empty; K/V zero so a read of an unwritten slot is well defined
     rc = launch_fill_kv(ctx, ctx->ring_k, (int64_t)(ctx->ring_bytes / kv_elem_bytes(ctx)), 0.f);
     if (rc) break;
@@ -251,6 +276,7 @@ void mb_destroy(mb_ctx* ctx) {
   (void)hipFree(ctx->ring_v);
   (void)hipFree(ctx->slot_pos);
   (void)hipFree(ctx->rope_tab);
+  (void)hipFree(ctx->split_part);
   for (void* p : {(void*)ctx->local_k, (void*)ctx->local_v, (void*)ctx->local_sp,
                   (void*)ctx->local_pos, (void*)ctx->seen, (void*)ctx->tokens, (void*)ctx->cont})
     (void)hipFree(p);
@@ -274,6 +300,7 @@ int mb_synchronize(mb_ctx* ctx) {
   MB_DEVICE_GUARD(ctx);
   if (!ctx) return MB_ERR_ARG;
   MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  release_split(ctx);
   return MB_OK;
 }
 
@@ -507,7 +534,7 @@ int mb_decode_attention_dev(mb_ctx* ctx, int layer, int B, const float* q, int64
   if (B == 0) return MB_OK;
   if (!q || !pos || !out) return fail(ctx, MB_ERR_ARG, "null pointer");
   return launch_attn(ctx, global_ring(ctx, layer), B, 1, q, dense_rows(q_stride, 1), pos, nullptr,
-                     (int64_t)max_pos + 1, out, dense_rows(out_stride, 1));
+                     (int64_t)max_pos + 1, out, dense_rows(out_stride, 1), claim_split(ctx));
 }
 
 int mb_append_attend_dev(mb_ctx* ctx, int layer, int B, const void* qkv, int qkv_dtype,
@@ -530,7 +557,8 @@ int mb_append_attend_dev(mb_ctx* ctx, int layer, int B, const void* qkv, int qkv
   if (!qkv || !pos || !out) return fail(ctx, MB_ERR_ARG, "null pointer");
   return launch_append_attn(ctx, global_ring(ctx, layer), B, qkv, qkv_dtype,
                             dense_rows(qkv_stride, 1), pos, (int64_t)max_pos + 1, q_out,
-                            dense_rows(q_stride, 1), out, dense_rows(out_stride, 1));
+                            dense_rows(q_stride, 1), out, dense_rows(out_stride, 1), -1,
+                            claim_split(ctx));
 }
 
 int mb_prefill_attention_dev(mb_ctx* ctx, int layer, int B, int rows_max, const void* q,
@@ -657,10 +685,11 @@ int mb_decode_attention(mb_ctx* ctx, int layer, int B, const float* q, const int
   MB_HIP(ctx, hipMemcpyAsync(d_q, q, (size_t)B * D * 4, hipMemcpyHostToDevice, ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(d_pos, pos, (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
   rc = launch_attn(ctx, global_ring(ctx, layer), B, 1, d_q, dense_rows(D, 1), d_pos, nullptr,
-                   (int64_t)max_pos + 1, d_out, dense_rows(D, 1));
+                   (int64_t)max_pos + 1, d_out, dense_rows(D, 1), claim_split(ctx));
   if (rc) return rc;
   MB_HIP(ctx, hipMemcpyAsync(out, d_out, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  release_split(ctx);
   return MB_OK;
 }
 
@@ -684,11 +713,12 @@ int mb_append_attend(mb_ctx* ctx, int layer, int B, const float* qkv, const int3
   MB_HIP(ctx, hipMemcpyAsync(d_pos, pos, (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
   rc = launch_append_attn(ctx, global_ring(ctx, layer), B, d_qkv, MB_DT_F32, dense_rows(QKV, 1),
                           d_pos, (int64_t)max_pos + 1, q_out ? d_q : nullptr, dense_rows(D, 1),
-                          d_out, dense_rows(D, 1));
+                          d_out, dense_rows(D, 1), -1, claim_split(ctx));
   if (rc) return rc;
   if (q_out) MB_HIP(ctx, hipMemcpyAsync(q_out, d_q, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(out, d_out, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  release_split(ctx);
   return MB_OK;
 }
 

@@ -133,6 +133,14 @@ struct mb_ctx {
   int32_t* slot_pos = nullptr;
   size_t ring_bytes = 0;  // bytes of ring_k (== ring_v)
 
+  // The kernel-level attention calls' AttnSplit (mb_create).  It is used by
+  // one stream at a time: the first call after the last synchronising one
+  // claims it (claim_split), calls on other streams run without.
+  float* split_part = nullptr;
+  int32_t* split_count = nullptr;
+  bool split_claimed = false;
+  hipStream_t split_stream = nullptr;
+
   // RoPE cos/sin for positions [0, kRopeTab): (cos, sin) of pair i at
   // position p in rope_tab[p * 32 + i]; later positions are computed in-kernel.
   float2* rope_tab = nullptr;
@@ -277,20 +285,32 @@ int launch_ring_write(mb_ctx* ctx, const RingView& ring, int B, int rows_max, co
 // run their attention as per-wave partials merged by the O projection
 // (launch_append_attn_parts, launch_gemv_k_parts).
 constexpr int kPartsMaxSeqs = 8;
+// Workspace of a decode attention whose (sequence, head) units are shared
+// between waves on different CUs (k_attn_unit's MERGE form): per unit
+// kSplitMaxWaves states and a counter that is zero between launches.  Calls
+// that use one must not overlap; with a null `part` every unit is one
+// workgroup's.
+constexpr int kSplitMaxUnits = 192, kSplitMaxWaves = 16;
+constexpr size_t kSplitFloats = (size_t)kSplitMaxUnits * kSplitMaxWaves * PART;
+struct AttnSplit {
+  float* part = nullptr;
+  int32_t* count = nullptr;
+};
 int launch_append_attn_parts(mb_ctx* ctx, const RingView& ring, int B, const float* qkv,
                              const int32_t* pos, int64_t max_valid, float* part, int& nw_out);
 int launch_gemv_k_parts(mb_ctx* ctx, int epi, const float* part, int nwp, const uint16_t* Wk,
                         int N, const float* bias, float* Cm, int64_t ldc, int M);
 int launch_attn(mb_ctx* ctx, const RingView& ring, int B, int rows, const float* q,
                 const Rows& q_rows, const int32_t* pos0, const int32_t* n_rows, int64_t max_valid,
-                float* out, const Rows& out_rows);
+                float* out, const Rows& out_rows, const AttnSplit& ws = {});
 // Ring append fused into the decode attention: one row per sequence, qkv
 // [B] fused rows at pos[b]; q_out (roped q) may be null.
 // pos_const >= 0: every row sits at that position (pos is then not read
 // where the kernel can skip it: the short-window fp32 ring of the local head).
 int launch_append_attn(mb_ctx* ctx, const RingView& ring, int B, const void* qkv, int qkv_dtype,
                        const Rows& qkv_rows, const int32_t* pos, int64_t max_valid, float* q_out,
-                       const Rows& qo_rows, float* out, const Rows& out_rows, int pos_const = -1);
+                       const Rows& qo_rows, float* out, const Rows& out_rows, int pos_const = -1,
+                       const AttnSplit& ws = {});
 int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                              const void* q, int q_dtype, const Rows& q_rows, const int32_t* pos0,
                              const int32_t* n_rows, float* out, const Rows& out_rows,

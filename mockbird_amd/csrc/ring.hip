@@ -10,6 +10,7 @@
 
 #include "mb_internal.h"
 #include "kv_types.h"
+#include "coherent.h"
 #include "rope.h"
 
 namespace mb {
@@ -303,14 +304,20 @@ __device__ __forceinline__ uint4 pack16(const float* x) {
 // acc[64], max, sum -- to out[(unit * nwp + wave) * PART] instead of folding
 // through LDS; the next projection merges them as it reads its input
 // (k_gemv_k's PIN form).
+//
+// MERGE (PARTS for calls that need the row itself): the wave that counts in
+// last on its unit's counter adds the unit's states and writes the row.  The
+// waves of a unit run on different XCDs, so states and counter move by
+// agent-scope accesses, as stream_finish's split tiles do; the last wave sets
+// the counter back to zero.
 template <bool KV_BF16, int U, int MAXNW, bool APPEND, bool IN_BF16, bool EARLY = false,
-          bool PARTS = false>
+          bool PARTS = false, bool MERGE = false>
 __global__ __launch_bounds__(64 * MAXNW, !KV_BF16 && APPEND ? 3 : 1) void k_attn_unit(
     const void* __restrict__ q, Rows q_rows, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ n_rows, int rows, void* __restrict__ ring_k,
     void* __restrict__ ring_v, int32_t* __restrict__ slot_pos, int64_t ring_seq_stride, int C,
     int wrap, const float2* __restrict__ rope_tab, float* __restrict__ q_out, Rows qo_rows,
-    float* __restrict__ out, Rows out_rows, int nwp) {
+    float* __restrict__ out, Rows out_rows, int nwp, AttnSplit ws = {}) {
   constexpr int VD = KV_BF16 ? 8 : 4;
   constexpr int LR = 64 / VD;
   constexpr int G = VD;
@@ -538,7 +545,41 @@ __global__ __launch_bounds__(64 * MAXNW, !KV_BF16 && APPEND ? 3 : 1) void k_attn
     for (int i = 0; i < VD; i++) ao[i] = __shfl_xor(acc[i], off);
     merge_state<VD>(m, l, acc, mo, lo, ao);
   }
-  if constexpr (PARTS) {
+  if constexpr (MERGE) {
+    float* const up = ws.part + (int64_t)unit * kSplitMaxWaves * PART;
+    if (g == 0) {
+      float* pp = up + wave * PART;
+#pragma unroll
+      for (int i = 0; i < VD; i += 2) store_coherent(pp + sub * VD + i, acc[i], acc[i + 1]);
+      if (sub == 0) store_coherent(pp + 64, m, l);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0): this wave's state is stored
+    int before = 0;
+    if (lane == 0)
+      before = __hip_atomic_fetch_add(&ws.count[unit], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(before) != nwp - 1) return;
+    asm volatile("" ::: "memory");  // the states are read after the count
+    // lane w holds wave w's (max, sum); every lane its dim of every state, the
+    // ones past nwp read again with weight 0
+    float ms, ls, o = 0.f, v[kSplitMaxWaves];
+    load_coherent(up + min(lane, nwp - 1) * PART + 64, ms, ls);
+#pragma unroll
+    for (int s = 0; s < kSplitMaxWaves; s++)
+      v[s] = __hip_atomic_load(up + min(s, nwp - 1) * PART + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane >= nwp) ms = -INFINITY;
+    float M = ms;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
+    const float w = (ms == -INFINITY) ? 0.f : __expf(ms - M);
+    float L = ls * w;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
+#pragma unroll
+    for (int s = 0; s < kSplitMaxWaves; s++) o = fmaf(__shfl(w, s), v[s], o);
+    out[row_at(out_rows, b, r) + head * HD + lane] = L > 0.f ? o / L : 0.f;
+    if (lane == 0) __hip_atomic_store(&ws.count[unit], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  } else if constexpr (PARTS) {
     if (g == 0) {
       float* pp = out + ((int64_t)unit * nwp + wave) * PART;
 #pragma unroll
@@ -752,11 +793,31 @@ static int unit_waves(int64_t max_valid, int per_wave, int maxnw) {
   return (int)std::min<int64_t>(maxnw, std::max(short_rule, long_rule));
 }
 
+// Waves that share a unit's window in the MERGE form, each a workgroup of its
+// own; 0: the one-workgroup form.  A few units leave most CUs idle and each
+// workgroup is a chain of dependent batches, so the split pays once the
+// window has enough batches for the units there are; with 16 voices' fp32
+// windows the chip is busy and it only adds the merge.  Twelve layers' fused
+// launches, one workgroup -> split, us: fp32 1 voice 512 / 1024 / 4096 slots
+// 104 -> 81, 164 -> 89, 458 -> 154; 4 voices 512 / 1024 / 2048 108 -> 97, 172
+// -> 120, 266 -> 147; 8 voices 384 / 1024 / 4096 103 -> 102, 182 -> 154, 548 ->
+// 362; 16 voices 1024 / 4096 221 -> 253, 668 -> 738.  bf16 1 voice 1024 / 4096
+// 120 -> 89, 273 -> 152; 8 voices 1024 / 2048 134 -> 134, 200 -> 164; 16 voices
+// 1024 / 2048 154 -> 191, 354 -> 238.  24 waves per unit were no better (1
+// voice 1024 slots 96 us, 4 voices 135).
+static int split_waves(const AttnSplit& ws, bool bf16, int64_t units, int64_t max_valid, int gu) {
+  const int64_t batches = (max_valid + gu - 1) / gu;
+  if (!ws.part || units > (bf16 ? kSplitMaxUnits : kSplitMaxUnits / 2) ||
+      batches < std::max<int64_t>(8, units / 5))
+    return 0;
+  return (int)std::min<int64_t>(kSplitMaxWaves, batches);
+}
+
 template <bool APPEND, bool IN_BF16>
 static int launch_unit(mb_ctx* ctx, const RingView& ring, int B, int rows, const void* q,
                        const Rows& q_rows, const int32_t* pos0, const int32_t* n_rows,
                        int64_t max_valid, float* q_out, const Rows& qo_rows, float* out,
-                       const Rows& out_rows, int pos_const = -1) {
+                       const Rows& out_rows, int pos_const = -1, const AttnSplit& ws = {}) {
   if (ring.heads != H || ring.window != ring.C)
     return fail(ctx, MB_ERR_ARG, "single-query decode attention runs on the model's 12-head rings");
   const int C = ring.C;
@@ -771,6 +832,24 @@ static int launch_unit(mb_ctx* ctx, const RingView& ring, int B, int rows, const
                        ctx->stream, q, q_rows, pos0, nunits, (float*)ring.k, (float*)ring.v,
                        ring.sp, ring.seq_stride, C, ctx->rope_tab, q_out, qo_rows, out, out_rows,
                        pos_const);
+    MB_HIP(ctx, hipGetLastError());
+    return MB_OK;
+  }
+  if (const int nwp = rows == 1 && !n_rows
+                          ? split_waves(ws, ring.bf16, nq * H, max_valid, ring.bf16 ? (max_valid <= kAttnShortWindow ? 64 : 32) : 48)
+                          : 0) {
+    const dim3 grid((unsigned)(nq * H * nwp));
+    auto go = [&](auto bf_, auto u_) {
+      hipLaunchKernelGGL((k_attn_unit<decltype(bf_)::value, decltype(u_)::value, 1, APPEND, IN_BF16, false,
+                                      true, true>),
+                         grid, dim3(64), 0, ctx->stream, q, q_rows, pos0, n_rows, rows, ring.k, ring.v,
+                         ring.sp, ring.seq_stride, C, ring.wrap, ctx->rope_tab, q_out, qo_rows, out,
+                         out_rows, nwp, ws);
+    };
+    using std::integral_constant;
+    if (!ring.bf16) go(std::false_type{}, integral_constant<int, 12>{});
+    else if (max_valid <= kAttnShortWindow) go(std::true_type{}, integral_constant<int, 8>{});
+    else go(std::true_type{}, integral_constant<int, 4>{});
     MB_HIP(ctx, hipGetLastError());
     return MB_OK;
   }
@@ -812,9 +891,9 @@ static int launch_unit(mb_ctx* ctx, const RingView& ring, int B, int rows, const
 
 int launch_attn(mb_ctx* ctx, const RingView& ring, int B, int rows, const float* q,
                 const Rows& q_rows, const int32_t* pos0, const int32_t* n_rows, int64_t max_valid,
-                float* out, const Rows& out_rows) {
+                float* out, const Rows& out_rows, const AttnSplit& ws) {
   return launch_unit<false, false>(ctx, ring, B, rows, q, q_rows, pos0, n_rows, max_valid, nullptr,
-                                   Rows{}, out, out_rows);
+                                   Rows{}, out, out_rows, -1, ws);
 }
 
 // The appended decode step of B <= kPartsMaxSeqs sequences as per-wave
@@ -855,12 +934,13 @@ int launch_append_attn_parts(mb_ctx* ctx, const RingView& ring, int B, const flo
 
 int launch_append_attn(mb_ctx* ctx, const RingView& ring, int B, const void* qkv, int qkv_dtype,
                        const Rows& qkv_rows, const int32_t* pos, int64_t max_valid, float* q_out,
-                       const Rows& qo_rows, float* out, const Rows& out_rows, int pos_const) {
+                       const Rows& qo_rows, float* out, const Rows& out_rows, int pos_const,
+                       const AttnSplit& ws) {
   if (qkv_dtype == MB_DT_BF16)
     return launch_unit<true, true>(ctx, ring, B, 1, qkv, qkv_rows, pos, nullptr, max_valid, q_out,
-                                   qo_rows, out, out_rows, pos_const);
+                                   qo_rows, out, out_rows, pos_const, ws);
   return launch_unit<true, false>(ctx, ring, B, 1, qkv, qkv_rows, pos, nullptr, max_valid, q_out,
-                                  qo_rows, out, out_rows, pos_const);
+                                  qo_rows, out, out_rows, pos_const, ws);
 }
 
 }  // namespace mb

@@ -389,6 +389,55 @@ def test_few_units_long_windows(name, kv):
         _check_ring(fused, ring, 0, range(B))
 
 
+@pytest.mark.parametrize("name,kv", KV)
+@pytest.mark.parametrize("B,C", [(1, 385), (1, 1000), (4, 530), (8, 1030)])
+def test_units_shared_between_waves(name, kv, B, C):
+    """Few units over windows of many batches: each (query, head) unit is
+    shared by up to 16 one-wave workgroups and merged by the last.  Windows
+    of one slot (waves without a batch), part full and wrapped, a strided
+    output; the same bits on every call, within fp32 rounding (1e-6 of O(1)
+    outputs: sums of up to 1030 weights in another order) of the same call on
+    a stream that does not hold the workspace."""
+    torch = pytest.importorskip("torch")
+    say(f"shared units kv={name} B={B} C={C}")
+    rng = np.random.default_rng([B, C])
+    pos = rng.integers(C // 2, 3 * C, size=B).astype(np.int32)
+    pos[0] = 0 if C == 385 else 2 * C + 3
+    dev = torch.device("cuda")
+    with mb.Context(n_layers=1, capacity=C, max_seqs=B, max_rows=C, kv_dtype=kv) as ctx:
+        ring = _oracle_ring(B, C, kv)
+        start = np.maximum(0, pos - C + 1).astype(np.int32)
+        n = (pos - start).astype(np.int32)
+        fill = rng.standard_normal((B, max(1, int(n.max())), 2304), dtype=np.float32)
+        ctx.ring_write_rows(0, fill, start, n)
+        ring.write(fill, start, n)
+        qkv = rng.standard_normal((B, 2304), dtype=np.float32)
+        q_or = ring.append(qkv, pos)
+        want = ring.attend(q_or, pos)
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        x, p = torch.from_numpy(qkv).to(dev), torch.from_numpy(pos).to(dev)
+        out = torch.zeros((5, B, 832), device=dev)
+        for i in range(3):
+            ctx.append_attend_dev(0, B, x.data_ptr(), p.data_ptr(), int(max(pos.max(), C)),
+                                  out[i].data_ptr(), out_stride=832)
+        q = torch.from_numpy(q_or).to(dev)
+        ctx.decode_attention_dev(0, B, q.data_ptr(), p.data_ptr(), int(max(pos.max(), C)),
+                                 out[3].data_ptr(), out_stride=832)
+        torch.cuda.synchronize()
+        other = torch.cuda.Stream()
+        ctx.set_stream(other.cuda_stream)  # the workspace still belongs to the first stream
+        ctx.append_attend_dev(0, B, x.data_ptr(), p.data_ptr(), int(max(pos.max(), C)),
+                              out[4].data_ptr(), out_stride=832)
+        other.synchronize()
+        got = out.cpu().numpy()
+        _check_ring(ctx, ring, 0, range(B))
+    for i in range(1, 4):
+        assert np.array_equal(got[i], got[0]), i
+    assert not got[:, :, 768:].any()
+    assert np.abs(got[4] - got[0]).max() < 1e-6
+    assert np.abs(got[0, :, :768] - want).max() < (2e-6 if kv == mb.MB_KV_F32 else 1e-4)
+
+
 def test_append_attend_range_error_on_a_non_wrapping_ring():
     say("fused append+attention range error")
     import torch
