@@ -1481,14 +1481,18 @@ static int gemv_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, const 
 // sums x - x0 and (x - x0)^2 over the rows it loads (x0 = x[m][0]) and
 // applies the folded LayerNorm itself.  The grid is N / 4 workgroups (192
 // for 768 outputs, 768 for 3072), and every output is a fixed-order sum.
-// KC > 0: K == KC known at compile time, so every round of loads is a fixed
-// set of unconditional loads (no branch around a load: the compiler then
-// leaves them in flight across the epilogue operands' waits); KC = 0: any K,
-// in a run-time loop.
+// K == KC (768 or 3072, all the model has) is known at compile time, so every
+// round of loads is a fixed set of unconditional loads (no branch around a
+// load: the compiler then leaves them in flight across the epilogue operands'
+// waits).  A run-time k loop in rounds of RI steps, as 2 to 8 rows had it,
+// also read and multiplied 12 (2 rows) or 6 (3-4 rows) steps where 768
+// columns have 3: four frames of 2 / 4 / 8 voices 4149 / 4505 / 5280 us against
+// 3163 / 3746 / 5007 this way (bf16 weights, k_gemv_k16: 4578 / 4593 / 6630 against
+// 3076 / 3969 / 5613).
 // (At most 4 waves per SIMD are asked for: a grid is N / 4 workgroups, one
 // column per wave, so at 768 and 3072 columns there are 0.75 and 3 waves per
 // SIMD, and the registers go to keeping every load of a round in flight.)
-template <int EPI, bool LNF, int MR, int KC = 0, bool PICK = false>
+template <int EPI, bool LNF, int MR, int KC, bool PICK = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_gemv_k(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ Wk, int N, int K,
     const float* __restrict__ bias, float* __restrict__ Cm, int64_t ldc, int M,
@@ -1517,7 +1521,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     x0[m] = LNF && !PICK ? A[(int64_t)min(m, M - 1) * lda] : 0.f;
   }
   const float* Ar = A;  // PICK: the chosen code's embedding row
-  const int Kx = KC > 0 ? KC : K;  // a constant where the launch fixed it
+  constexpr int Kx = KC;  // == K
   // one k step (256 k): lane l's float4 at k = 256 step + 4 l.  Lanes past K
   // (only in a last, partial step) add zeros: no branch, so no load is sunk
   // into one.
@@ -1552,42 +1556,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     load_w(st, w);
     load_a(st, a);
   };
-  if constexpr (KC > 0) {
-    constexpr int SPR = (KC + 255) / 256;
-    constexpr int RK = SPR < RI ? SPR : RI;
-    static_assert(!PICK || RK == SPR, "PICK: one round of loads");
-    static_for<(SPR + RK - 1) / RK>([&](auto r_) {
-      constexpr int r = decltype(r_)::value;
-      constexpr int NI = (r + 1) * RK <= SPR ? RK : SPR - r * RK;
-      float4 w[NI], a[NI][MR];
-      if constexpr (PICK) {
-        // the choice's logits first, the weights behind them, then the
-        // choice (waiting for the logits only) and the chosen row
-        const ChoiceIn c = pick_load(pk, lane);
+  constexpr int SPR = (KC + 255) / 256;
+  constexpr int RK = SPR < RI ? SPR : RI;
+  static_assert(!PICK || RK == SPR, "PICK: one round of loads");
+  static_for<(SPR + RK - 1) / RK>([&](auto r_) {
+    constexpr int r = decltype(r_)::value;
+    constexpr int NI = (r + 1) * RK <= SPR ? RK : SPR - r * RK;
+    float4 w[NI], a[NI][MR];
+    if constexpr (PICK) {
+      // the choice's logits first, the weights behind them, then the
+      // choice (waiting for the logits only) and the chosen row
+      const ChoiceIn c = pick_load(pk, lane);
 #pragma unroll
-        for (int i = 0; i < NI; i++) load_w(i, w[i]);
-        Ar = pick_row(pk, c, lane, blockIdx.x == 0 && wave == 0);
-        x0[0] = Ar[0];
+      for (int i = 0; i < NI; i++) load_w(i, w[i]);
+      Ar = pick_row(pk, c, lane, blockIdx.x == 0 && wave == 0);
+      x0[0] = Ar[0];
 #pragma unroll
-        for (int i = 0; i < NI; i++) load_a(i, a[i]);
-      } else {
+      for (int i = 0; i < NI; i++) load_a(i, a[i]);
+    } else {
 #pragma unroll
-        for (int i = 0; i < NI; i++) step_load(r * RK + i, w[i], a[i]);
-      }
-      asm volatile("" ::: "memory");  // the round's loads stay in front, none sunk into a branch
-#pragma unroll
-      for (int i = 0; i < NI; i++) step_mac(r * RK + i, w[i], a[i]);
-    });
-  } else {
-    const int steps = (K + 255) >> 8;
-    for (int i0 = 0; i0 < steps; i0 += RI) {
-      float4 w[RI], a[RI][MR];
-#pragma unroll
-      for (int i = 0; i < RI; i++) step_load(i0 + i, w[i], a[i]);
-#pragma unroll
-      for (int i = 0; i < RI; i++) step_mac(i0 + i, w[i], a[i]);
+      for (int i = 0; i < NI; i++) step_load(r * RK + i, w[i], a[i]);
     }
-  }
+    asm volatile("" ::: "memory");  // the round's loads stay in front, none sunk into a branch
+#pragma unroll
+    for (int i = 0; i < NI; i++) step_mac(r * RK + i, w[i], a[i]);
+  });
   auto fold = [](float v) {
 #pragma unroll
     for (int sh = 1; sh < 16; sh <<= 1) v += __shfl_xor(v, sh);
@@ -1643,14 +1636,12 @@ int launch_gemv_k(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float
     MB_HIP(ctx, hipGetLastError());
     return MB_OK;
   }
-  if (M > kGemvMaxM || N % 4 || K % 4 || lda % 4 || ((uintptr_t)A & 15) || ((uintptr_t)Wk & 15) ||
-      (lnf && !lnd))
+  if (M > kGemvMaxM || N % 4 || (K != D && (K != FFN || lnf)) || lda % 4 || ((uintptr_t)A & 15) ||
+      ((uintptr_t)Wk & 15) || (lnf && !lnd))
     return fail(ctx, MB_ERR_ARG, "k-major gemv shape/alignment unsupported (M %d N %d K %d)", M, N, K);
   if (lnf && epi != EPI_STORE && epi != EPI_GELU && epi != EPI_GELU_ERF)
     return fail(ctx, MB_ERR_ARG, "folded LayerNorm gemm has no epilogue %d", epi);
   const dim3 grid((unsigned)(N / 4));
-  // one row at the model's two widths: k loops fixed at compile time
-  const int kc = M == 1 && (K == D || K == FFN) ? K : 0;
   with_epi(epi, [&](auto e) {
     constexpr int E = decltype(e)::value;
     auto go = [&](auto mr) {
@@ -1658,7 +1649,7 @@ int launch_gemv_k(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float
       auto launch = [&](auto kc_) {
         constexpr int KCv = decltype(kc_)::value;
         if (lnf) {
-          if constexpr (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF)
+          if constexpr (KCv == D && (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF))
             hipLaunchKernelGGL((k_gemv_k<E, true, MRv, KCv>), grid, dim3(256), 0, ctx->stream, A,
                                lda, Wk, N, K, bias, Cm, ldc, M, lnc, lnd, PickIn{});
         } else {
@@ -1666,11 +1657,8 @@ int launch_gemv_k(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float
                              lda, Wk, N, K, bias, Cm, ldc, M, lnc, lnd, PickIn{});
         }
       };
-      if constexpr (MRv == 1) {
-        if (kc == D) return launch(std::integral_constant<int, D>{});
-        if (kc == FFN) return launch(std::integral_constant<int, FFN>{});
-      }
-      launch(std::integral_constant<int, 0>{});
+      if (K == D) launch(std::integral_constant<int, D>{});
+      else launch(std::integral_constant<int, FFN>{});
     };
     if (M <= 1) go(std::integral_constant<int, 1>{});
     else if (M <= 2) go(std::integral_constant<int, 2>{});
@@ -1829,7 +1817,7 @@ int launch_gemv_k_parts(mb_ctx* ctx, int epi, const float* part, int nwp, const 
 // contiguous per load), with the matching two float4 of every A row (and of
 // gamma with GAM), all issued before the first multiply-add.  The LayerNorm
 // sums of LNF are taken over the raw rows, as in k_gemv_k.
-template <int EPI, bool LNF, bool GAM, int MR, int KC = 0, bool PICK = false>
+template <int EPI, bool LNF, bool GAM, int MR, int KC, bool PICK = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) void k_gemv_k16(
     const float* __restrict__ A, int64_t lda, const uint16_t* __restrict__ Wk, int N, int K,
     const float* __restrict__ bias, float* __restrict__ Cm, int64_t ldc, int M,
@@ -1856,7 +1844,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
     x0[m] = LNF && !PICK ? A[(int64_t)min(m, M - 1) * lda] : 0.f;
   }
   const float* Ar = A;  // PICK: the chosen code's embedding row
-  const int Kx = KC > 0 ? KC : K;  // a constant where the launch fixed it
+  constexpr int Kx = KC;  // == K
   auto load_w = [&](int st, uint4& w, float4* g) {
     const int k = min(st * 512 + 8 * lane, Kx - 8);
     w = *(const uint4*)(wp + k);
@@ -1907,43 +1895,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
       }
     }
   };
-  if constexpr (KC > 0) {
-    constexpr int SPR = (KC + 511) / 512;
-    constexpr int RK = SPR < RI ? SPR : RI;
-    static_assert(!PICK || RK == SPR, "PICK: one round of loads");
-    static_for<(SPR + RK - 1) / RK>([&](auto r_) {
-      constexpr int r = decltype(r_)::value;
-      constexpr int NI = (r + 1) * RK <= SPR ? RK : SPR - r * RK;
-      uint4 w[NI];
-      float4 g[NI][2], a[NI][MR][2];
-      if constexpr (PICK) {
-        // as in k_gemv_k: the choice's logits, the weights, the choice, the row
-        const ChoiceIn c = pick_load(pk, lane);
+  constexpr int SPR = (KC + 511) / 512;
+  constexpr int RK = SPR < RI ? SPR : RI;
+  static_assert(!PICK || RK == SPR, "PICK: one round of loads");
+  static_for<(SPR + RK - 1) / RK>([&](auto r_) {
+    constexpr int r = decltype(r_)::value;
+    constexpr int NI = (r + 1) * RK <= SPR ? RK : SPR - r * RK;
+    uint4 w[NI];
+    float4 g[NI][2], a[NI][MR][2];
+    if constexpr (PICK) {
+      // as in k_gemv_k: the choice's logits, the weights, the choice, the row
+      const ChoiceIn c = pick_load(pk, lane);
 #pragma unroll
-        for (int i = 0; i < NI; i++) load_w(i, w[i], g[i]);
-        Ar = pick_row(pk, c, lane, blockIdx.x == 0 && wave == 0);
-        x0[0] = Ar[0];
+      for (int i = 0; i < NI; i++) load_w(i, w[i], g[i]);
+      Ar = pick_row(pk, c, lane, blockIdx.x == 0 && wave == 0);
+      x0[0] = Ar[0];
 #pragma unroll
-        for (int i = 0; i < NI; i++) load_a(i, a[i]);
-      } else {
+      for (int i = 0; i < NI; i++) load_a(i, a[i]);
+    } else {
 #pragma unroll
-        for (int i = 0; i < NI; i++) step_load(r * RK + i, w[i], g[i], a[i]);
-      }
-      asm volatile("" ::: "memory");  // the round's loads stay in front, none sunk into a branch
-#pragma unroll
-      for (int i = 0; i < NI; i++) step_mac(r * RK + i, w[i], g[i], a[i]);
-    });
-  } else {
-    const int steps = (K + 511) >> 9;
-    for (int i0 = 0; i0 < steps; i0 += RI) {
-      uint4 w[RI];
-      float4 g[RI][2], a[RI][MR][2];
-#pragma unroll
-      for (int i = 0; i < RI; i++) step_load(i0 + i, w[i], g[i], a[i]);
-#pragma unroll
-      for (int i = 0; i < RI; i++) step_mac(i0 + i, w[i], g[i], a[i]);
+      for (int i = 0; i < NI; i++) step_load(r * RK + i, w[i], g[i], a[i]);
     }
-  }
+    asm volatile("" ::: "memory");  // the round's loads stay in front, none sunk into a branch
+#pragma unroll
+    for (int i = 0; i < NI; i++) step_mac(r * RK + i, w[i], g[i], a[i]);
+  });
   auto fold = [](float v) {
 #pragma unroll
     for (int sh = 1; sh < 16; sh <<= 1) v += __shfl_xor(v, sh);
@@ -2007,13 +1983,12 @@ int launch_gemv_k16(mb_ctx* ctx, int epi, const float* A, int64_t lda, const uin
     MB_HIP(ctx, hipGetLastError());
     return MB_OK;
   }
-  if (M > kGemvMaxM || N % 4 || K % 8 || lda % 4 || ((uintptr_t)A & 15) || ((uintptr_t)Wk & 15) ||
-      ((uintptr_t)gamma & 15) || (lnf && !lnd))
+  if (M > kGemvMaxM || N % 4 || (K != D && (K != FFN || lnf)) || lda % 4 || ((uintptr_t)A & 15) ||
+      ((uintptr_t)Wk & 15) || ((uintptr_t)gamma & 15) || (lnf && !lnd))
     return fail(ctx, MB_ERR_ARG, "bf16 k-major gemv shape/alignment unsupported (M %d N %d K %d)", M, N, K);
   if (lnf && epi != EPI_STORE && epi != EPI_GELU && epi != EPI_GELU_ERF)
     return fail(ctx, MB_ERR_ARG, "folded LayerNorm gemm has no epilogue %d", epi);
   const dim3 grid((unsigned)(N / 4));
-  const int kc = M == 1 && (K == D || K == FFN) ? K : 0;  // as launch_gemv_k
   with_epi(epi, [&](auto e) {
     constexpr int E = decltype(e)::value;
     auto go = [&](auto mr) {
@@ -2021,7 +1996,7 @@ int launch_gemv_k16(mb_ctx* ctx, int epi, const float* A, int64_t lda, const uin
       auto launch = [&](auto kc_) {
         constexpr int KCv = decltype(kc_)::value;
         if (lnf) {
-          if constexpr (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF) {
+          if constexpr (KCv == D && (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF)) {
             if (gamma)
               hipLaunchKernelGGL((k_gemv_k16<E, true, true, MRv, KCv>), grid, dim3(256), 0,
                                  ctx->stream, A, lda, Wk, N, K, bias, Cm, ldc, M, lnc, lnd, gamma,
@@ -2037,11 +2012,8 @@ int launch_gemv_k16(mb_ctx* ctx, int epi, const float* A, int64_t lda, const uin
                              PickIn{});
         }
       };
-      if constexpr (MRv == 1) {
-        if (kc == D) return launch(std::integral_constant<int, D>{});
-        if (kc == FFN) return launch(std::integral_constant<int, FFN>{});
-      }
-      launch(std::integral_constant<int, 0>{});
+      if (K == D) launch(std::integral_constant<int, D>{});
+      else launch(std::integral_constant<int, FFN>{});
     };
     if (M <= 1) go(std::integral_constant<int, 1>{});
     else if (M <= 2) go(std::integral_constant<int, 2>{});
