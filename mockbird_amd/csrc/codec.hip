@@ -186,6 +186,18 @@ RingView codec_ring(const mb_ctx* ctx, const CodecState& cs, int layer, int stag
   return v;
 }
 
+// The codec's projections (N and K of 192 .. 1024): up to 3 rows on the GEMV
+// kernel, from 4 on the streaming one.  A workgroup of the first is 16 columns
+// over all of k, and its time grows with the rows: 5.3 / 7.0 us at 4 / 8 rows
+// where a streaming launch of up to 16 rows takes 4.2 (K = 256) to 6.8 (K =
+// 1024).  Per 4-frame call, GEMV up to 8 / 4 / 3 rows: 1 voice 1892 / 1808 /
+// 1784 us, 2 voices 1922 / 1779 / 1779 (bf16 rings 1728 / 1645 / 1625).
+constexpr int kCodecGemvRows = 3;
+int gemm(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float* W, int N, int K,
+         const float* bias, float* C, int64_t ldc, int M) {
+  return launch_gemm(ctx, epi, A, lda, W, N, K, bias, C, ldc, M, false, nullptr, 0, kCodecGemvRows);
+}
+
 int cancelled(mb_ctx* ctx) {
   if (ctx->cancel.load()) return fail(ctx, MB_ERR_CANCELLED, "cancelled");
   return MB_OK;
@@ -375,7 +387,7 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
   hipLaunchKernelGGL(k_rvq_accum, dim3((unsigned)(((int64_t)B * kRvq + 255) / 256)), dim3(256), 0,
                      ctx->stream, codes, cs.frame, B, cs.rvq_w, cs.rvq_b, cs.rvq_book, cs.acc);
   MB_HIP(ctx, hipGetLastError());
-  if ((rc = launch_gemm(ctx, EPI_STORE, cs.acc, kRvq, cs.rvq_out, kRvqOut, kRvq, cs.rvq_out_b,
+  if ((rc = gemm(ctx, EPI_STORE, cs.acc, kRvq, cs.rvq_out, kRvqOut, kRvq, cs.rvq_out_b,
                         cs.wide, kRvqOut, B)))
     return rc;
   int in_w = 192;
@@ -384,7 +396,7 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
     const CodecStageW& st = cs.stages[s];
     int32_t* pos = cs.pos + (int64_t)s * V;
     const int32_t* nrow = cs.nrow + (int64_t)s * V;
-    if ((rc = launch_gemm(ctx, EPI_STORE, cs.wide, in_w, st.in_proj, kD, in_w, nullptr, cs.x, kD, M)))
+    if ((rc = gemm(ctx, EPI_STORE, cs.wide, in_w, st.in_proj, kD, in_w, nullptr, cs.x, kD, M)))
       return rc;
     for (int i = 0; i < cs.cfg.layers[s]; i++) {
       const CodecLayerW& w = st.layers[i];
@@ -401,9 +413,9 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
                                 3 * kD, M, w.qkv_c, w.qkv_d);
         if (fold_qkv)
           return launch_gemm_ln(ctx, EPI_STORE, cs.x, kD, w.qkv_g, 3 * kD, kD, w.qkv_c, w.qkv_d,
-                                nullptr, cs.qkv, 3 * kD, M);
+                                nullptr, cs.qkv, 3 * kD, M, kCodecGemvRows);
         int r = launch_layernorm(ctx, cs.x, kD, nullptr, M, w.ln1_w, w.ln1_b, cs.h, kD, kD);
-        return r ? r : launch_gemm(ctx, EPI_STORE, cs.h, kD, w.qkv, 3 * kD, kD, nullptr, cs.qkv, 3 * kD, M);
+        return r ? r : gemm(ctx, EPI_STORE, cs.h, kD, w.qkv, 3 * kD, kD, nullptr, cs.qkv, 3 * kD, M);
       };
       auto f1_proj = [&]() {
         if (x3)
@@ -411,24 +423,24 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
                                 kFfn, M, w.f1_c, w.f1_d);
         if (fold_f1)
           return launch_gemm_ln(ctx, EPI_GELU_ERF, cs.x, kD, w.f1_g, kFfn, kD, w.f1_c, w.f1_d,
-                                nullptr, cs.ffn, kFfn, M);
+                                nullptr, cs.ffn, kFfn, M, kCodecGemvRows);
         int r = launch_layernorm(ctx, cs.x, kD, nullptr, M, w.ln2_w, w.ln2_b, cs.h, kD, kD);
-        return r ? r : launch_gemm(ctx, EPI_GELU_ERF, cs.h, kD, w.f1, kFfn, kD, nullptr, cs.ffn, kFfn, M);
+        return r ? r : gemm(ctx, EPI_GELU_ERF, cs.h, kD, w.f1, kFfn, kD, nullptr, cs.ffn, kFfn, M);
       };
       if ((rc = qkv_proj()) ||
           (rc = launch_window_attention(ctx, ring, B, n, cs.qkv, dense_rows(3 * kD, n), pos, nrow,
                                         cs.att, dense_rows(kD, n), cs.part)) ||
           (rc = x3 ? launch_gemm_x3(ctx, EPI_SCALE_ADD, cs.att, kD, w.o_x, kD, kD, w.s1, cs.x, kD,
                                       M, nullptr, nullptr)
-                     : launch_gemm(ctx, EPI_SCALE_ADD, cs.att, kD, w.o, kD, kD, w.s1, cs.x, kD, M)) ||
+                     : gemm(ctx, EPI_SCALE_ADD, cs.att, kD, w.o, kD, kD, w.s1, cs.x, kD, M)) ||
           (rc = f1_proj()) ||
           (rc = x3 ? launch_gemm_x3(ctx, EPI_SCALE_ADD, cs.ffn, kFfn, w.f2_x, kD, kFfn, w.s2, cs.x,
                                       kD, M, nullptr, nullptr)
-                     : launch_gemm(ctx, EPI_SCALE_ADD, cs.ffn, kFfn, w.f2, kD, kFfn, w.s2, cs.x, kD, M)))
+                     : gemm(ctx, EPI_SCALE_ADD, cs.ffn, kFfn, w.f2, kD, kFfn, w.s2, cs.x, kD, M)))
         return rc;
     }
     const int out_w = s == kStages - 1 ? kD : kRvqOut;
-    if ((rc = launch_gemm(ctx, EPI_STORE, cs.x, kD, st.out_proj, out_w, kD, nullptr, cs.wide, out_w, M)))
+    if ((rc = gemm(ctx, EPI_STORE, cs.x, kD, st.out_proj, out_w, kD, nullptr, cs.wide, out_w, M)))
       return rc;
     in_w = 384;
   }

@@ -411,18 +411,26 @@ __device__ __forceinline__ void stream_finish(f32x4_t (&acc)[MI][4], float (&sx)
 // x - x0 and (x - x0)^2 with x0 = x[row][0], so the variance does not cancel
 // -- which requires the workgroup to see the whole row (S == 1, K == 768).
 //
-// PLANES: the products on the bf16 matrix unit.  A wave splits the A rows and
+// ALT with tiles of 32 rows and more (PLANES): the products on the bf16
+// matrix unit.  A wave splits the A rows and
 // W columns it holds into three exact bf16 planes each (planes.h) and sums the
 // six plane products above 2^-24 in fp32: per 16 x 16 x 32 block 6 MFMAs of 16
 // cycles in place of 8 of 32.  Its error against float64 is the smaller one
 // (768-deep 2.5e-7 -> 2.1e-7, 3072-deep 5.0e-7 -> 4.3e-7 relative: fewer
 // roundings of the running sum).  stream_planes says where it is taken.
-template <int MT, int ST, int EPI, bool LNF, bool TILED, bool PLANES>
+//
+// ALT with 16-row tiles (the codec's, launch_gemm's gemv_rows): the two stages
+// are summed apart, with half as many roundings of a running sum.  That keeps
+// the error of a voice's codec frame, whose 4 and 8 rows the GEMV kernel took
+// before, where it was (4.1e-7 relative; 4.3e-7 there, 5.0e-7 with one sum).
+// The model's launches keep one sum: two cost 2 % of a 12-voice frame.
+template <int MT, int ST, int EPI, bool LNF, bool TILED, bool ALT>
 __global__ __launch_bounds__(256) void k_gemm_stream(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ W, int N, int kw,
     const float* __restrict__ bias, float* __restrict__ Cm, int64_t ldc, int M,
     float* __restrict__ part, const float* __restrict__ lnc, const float* __restrict__ lnd) {
   constexpr int MI = MT / 16;
+  constexpr bool PLANES = ALT && MI > 1, APART = ALT && MI == 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, r = lane >> 4;
   const int n = blockIdx.x * 64 + 4 * l16;
@@ -448,6 +456,8 @@ __global__ __launch_bounds__(256) void k_gemm_stream(
   auto stream = [&](auto planes_) {
     constexpr bool PL = decltype(planes_)::value;
     constexpr int CD = PL ? 2 : 1, STEP = CD * kStreamChunk;
+    constexpr int NA = APART ? ST : 1;  // sums per output
+    f32x4_t more[NA][4] = {};
 #pragma unroll
     for (int i = 0; i < MI; i++) {
 #pragma unroll
@@ -507,8 +517,10 @@ __global__ __launch_bounds__(256) void k_gemm_stream(
 #pragma unroll
           for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st][i][0][t], w[st][t][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 4; j++) {
+              f32x4_t& c = NA > 1 && st > 0 ? more[st][j] : acc[i][j];
+              c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st][i][0][t], w[st][t][j], c, 0, 0, 0);
+            }
       }
     };
     // Prefetch ST - 1 steps, then per step: issue the load ST - 1 ahead and
@@ -534,6 +546,10 @@ __global__ __launch_bounds__(256) void k_gemm_stream(
 #pragma unroll
     for (int s = 0; s < ST - 1; s++)
       if (c + s < nc) mma(s);
+#pragma unroll
+    for (int s = 1; s < NA; s++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[0][j] += more[s][j];
   };
   if constexpr (PLANES) {
     stream(std::true_type{});
@@ -783,8 +799,8 @@ static bool stream_planes(int mt, int K, int kw) {
 template <int MT, int ST, bool LNF>
 static int stream_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float* W, int N,
                          int K, const float* bias, float* Cm, int64_t ldc, int M, int S,
-                         const float* lnc, const float* lnd, bool tiled, float* part_ext = nullptr,
-                         size_t part_cap = 0) {
+                         const float* lnc, const float* lnd, bool tiled, bool apart,
+                         float* part_ext = nullptr, size_t part_cap = 0) {
   const int tx = N / 64, ty = (M + MT - 1) / MT;
   float* part = nullptr;
   if (S > 1) {
@@ -801,7 +817,7 @@ static int stream_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, cons
   }
   dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)S);
   const int kw = K / (4 * S);
-  const bool planes = stream_planes(MT, K, kw);
+  const bool alt = MT > 16 ? stream_planes(MT, K, kw) : apart;
   if (LNF && epi != EPI_STORE && epi != EPI_GELU && epi != EPI_GELU_ERF)
     return fail(ctx, MB_ERR_ARG, "folded LayerNorm gemm has no epilogue %d", epi);
   with_epi(epi, [&](auto e) {
@@ -809,17 +825,17 @@ static int stream_launch(mb_ctx* ctx, int epi, const float* A, int64_t lda, cons
     // folded weights (LNF) always come tiled from launch_fold_ln
     if constexpr (LNF) {
       if constexpr (E == EPI_STORE || E == EPI_GELU || E == EPI_GELU_ERF)
-        hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, true, true, (MT > 16)>
+        hipLaunchKernelGGL((alt ? k_gemm_stream<MT, ST, E, true, true, true>
                                    : k_gemm_stream<MT, ST, E, true, true, false>),
                            grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part,
                            lnc, lnd);
     } else if (tiled) {
-      hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, false, true, (MT > 16)>
+      hipLaunchKernelGGL((alt ? k_gemm_stream<MT, ST, E, false, true, true>
                                  : k_gemm_stream<MT, ST, E, false, true, false>),
                          grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc,
                          lnd);
     } else {
-      hipLaunchKernelGGL((planes ? k_gemm_stream<MT, ST, E, false, false, (MT > 16)>
+      hipLaunchKernelGGL((alt ? k_gemm_stream<MT, ST, E, false, false, true>
                                  : k_gemm_stream<MT, ST, E, false, false, false>),
                          grid, dim3(256), 0, ctx->stream, A, lda, W, N, kw, bias, Cm, ldc, M, part, lnc,
                          lnd);
@@ -2228,20 +2244,21 @@ bool gemm_streams(int M, int N) {
 // MB_ERR_STATE, so the caller runs the LayerNorm and the GEMM apart.
 int launch_gemm_ln(mb_ctx* ctx, int epi, const float* x, int64_t ldx, const float* Wg, int N,
                    int K, const float* c, const float* d, const float* bias, float* Cm,
-                   int64_t ldc, int M) {
+                   int64_t ldc, int M, int gemv_rows) {
   if (M <= 0) return MB_OK;
   if (!gemm_streams(M, N)) return MB_ERR_STATE;
   if (K % 64 || N % 64 || ldx % 4 || ldc % 4 || ((uintptr_t)x & 15) || ((uintptr_t)Wg & 15) ||
       ((uintptr_t)Cm & 15) || ((uintptr_t)bias & 15) || ((uintptr_t)c & 15) || ((uintptr_t)d & 15))
     return fail(ctx, MB_ERR_ARG, "folded gemm shape/alignment unsupported (M %d N %d K %d)", M, N, K);
-  if (M <= kGemvMaxM) return gemv_launch<true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, true, c, d);
+  if (M <= gemv_rows) return gemv_launch<true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, true, c, d);
+  const bool apart = gemv_rows < kGemvMaxM;
   int mt, S;
   stream_shape(M, N, K, true, mt, S);
   switch (mt) {
-    case 16: return stream_launch<16, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true);
-    case 32: return stream_launch<32, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true);
-    case 48: return stream_launch<48, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true);
-    default: return stream_launch<64, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true);
+    case 16: return stream_launch<16, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true, apart);
+    case 32: return stream_launch<32, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true, apart);
+    case 48: return stream_launch<48, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true, apart);
+    default: return stream_launch<64, 2, true>(ctx, epi, x, ldx, Wg, N, K, bias, Cm, ldc, M, 1, c, d, true, apart);
   }
 }
 
@@ -2272,23 +2289,24 @@ size_t gemm_partial_floats(int M, int N, int K) {
 
 int launch_gemm(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float* W, int N, int K,
                 const float* bias, float* Cm, int64_t ldc, int M, bool w_tiled, float* part,
-                size_t part_cap) {
+                size_t part_cap, int gemv_rows) {
   if (M <= 0) return MB_OK;
   if (w_tiled && !gemm_streams(M, N))
     return fail(ctx, MB_ERR_STATE, "tiled weights need the streaming kernel (M %d N %d)", M, N);
   if (N % 64 || K % 64 || lda % 4 || ldc % 4 || ((uintptr_t)A & 15) ||
       ((uintptr_t)W & 15) || ((uintptr_t)Cm & 15) || ((uintptr_t)bias & 15))
     return fail(ctx, MB_ERR_ARG, "gemm shape/alignment unsupported (M %d N %d K %d)", M, N, K);
-  if (M <= kGemvMaxM)
+  if (M <= gemv_rows)
     return gemv_launch<false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, w_tiled, nullptr, nullptr);
   if (gemm_streams(M, N)) {
+    const bool apart = gemv_rows < kGemvMaxM;
     int mt, S;
     stream_shape(M, N, K, false, mt, S);
     switch (mt) {
-      case 16: return stream_launch<16, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, part, part_cap);
-      case 32: return stream_launch<32, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, part, part_cap);
-      case 48: return stream_launch<48, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, part, part_cap);
-      default: return stream_launch<64, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, part, part_cap);
+      case 16: return stream_launch<16, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, apart, part, part_cap);
+      case 32: return stream_launch<32, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, apart, part, part_cap);
+      case 48: return stream_launch<48, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, apart, part, part_cap);
+      default: return stream_launch<64, 2, false>(ctx, epi, A, lda, W, N, K, bias, Cm, ldc, M, S, nullptr, nullptr, w_tiled, apart, part, part_cap);
     }
   }
   auto blocks = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * (N / bn); };

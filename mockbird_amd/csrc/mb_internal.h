@@ -343,11 +343,13 @@ enum { EPI_STORE = 0, EPI_GELU = 1, EPI_ADD = 2, EPI_SCALE_ADD = 3, EPI_GELU_ERF
 // `part` (optional, part_cap floats) takes the streaming kernel's split-K
 // partials in place of the context's growable scratch; a split that needs
 // more is MB_ERR_ARG.  M <= kGemvMaxM rows take the GEMV kernel, which needs
-// no scratch.
+// no scratch (M <= gemv_rows where a caller with K < 2048, never split, knows
+// the streaming kernel to be faster above; its 16-row tiles then sum their
+// stages apart).
 constexpr int kGemvMaxM = 8;
 int launch_gemm(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float* W, int N, int K,
                 const float* bias, float* Cm, int64_t ldc, int M, bool w_tiled = false,
-                float* part = nullptr, size_t part_cap = 0);
+                float* part = nullptr, size_t part_cap = 0, int gemv_rows = kGemvMaxM);
 // Floats of split-K partials launch_gemm writes for an M x N x K projection
 // (0: no split).
 size_t gemm_partial_floats(int M, int N, int K);
@@ -379,7 +381,7 @@ int launch_fold_ln(mb_ctx* ctx, const float* W, int K, int N, const float* gamma
                    const float* beta, float* Wg, float* c, float* d);
 int launch_gemm_ln(mb_ctx* ctx, int epi, const float* x, int64_t ldx, const float* Wg, int N,
                    int K, const float* c, const float* d, const float* bias, float* Cm,
-                   int64_t ldc, int M);
+                   int64_t ldc, int M, int gemv_rows = kGemvMaxM);
 // Split-bf16 projections (bf16-KV contexts): Wx, 2 K N bf16 values, holds
 // each weight of an fp32 W -- column-block-major [N / 64][K][64] (tiled:
 // launch_tile_w, launch_fold_ln's Wg) or row-major [K][N] -- as a bf16 high
