@@ -765,6 +765,10 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
 //    into a bf16 high part and a bf16 remainder, two MFMAs each, so the
 //    products keep about 16 bits (the scores and weights agree with the fp32
 //    path to ~1e-5 relative) at an eighth of the fp32 MFMA time.
+//    q's parts are read from LDS at each group: held in registers (136 for
+//    32 queries) they left one workgroup per CU, now two run (119).  The fp32
+//    form keeps q in registers: from LDS it gains no workgroup and 256 voices
+//    took 14.84 against 14.75 ms per four frames.
 // Partials (max, sum, 64 dims per query) fold across the waves through LDS.
 // SPLIT: gridDim.z workgroups share one window, and each leaves its folded
 // state in `part` (k_window_merge adds them up).  Where a launch has few
@@ -788,7 +792,10 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
   constexpr int NQ = 16 * QB;
   __shared__ float red_ml[NW][2][NQ];        // per wave: max (log2 units), sum
   __shared__ float red_acc[NW][NQ][HD + 1];  // per wave: unnormalised output
-  __shared__ __align__(16) float q_l[NQ][HD];  // the chunk's roped q rows (this head)
+  // the chunk's roped q rows (this head): fp32, or for bf16 rings their bf16
+  // high parts and remainders, 8-dim chunks swizzled
+  __shared__ __align__(16) float q_l[KV_BF16 ? 1 : NQ][HD];
+  __shared__ __align__(16) uint16_t q_p[KV_BF16 ? 2 : 1][KV_BF16 ? NQ * HD : 8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int qc = lane & 15, g = lane >> 4;
   const int h = blockIdx.x, b = blockIdx.y;
@@ -910,46 +917,39 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
 #pragma unroll
         for (int e = 0; e < 8; e++) qo[e] = 0.f;
       }
-      *(float4*)&q_l[r][d0] = make_float4(qo[0], qo[1], qo[2], qo[3]);
-      *(float4*)&q_l[r][d0 + 4] = make_float4(qo[4], qo[5], qo[6], qo[7]);
+      if constexpr (KV_BF16) {
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) split2_pair(qo[2 * j], qo[2 * j + 1], hi[j], lo[j]);
+        *(uint4*)&q_p[0][swz(r, d0 >> 3)] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        *(uint4*)&q_p[1][swz(r, d0 >> 3)] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      } else {
+        *(float4*)&q_l[r][d0] = make_float4(qo[0], qo[1], qo[2], qo[3]);
+        *(float4*)&q_l[r][d0 + 4] = make_float4(qo[4], qo[5], qo[6], qo[7]);
+      }
     }
   }
   __threadfence_block();
   __syncthreads();  // the rows are in the ring and q in LDS for every wave
 
-  // the wave's first group is in flight while q is split
+  // the wave's first group is in flight while its state is set up
   if (g0 < groups && !early) load_group(g0, cur);
   // Positions relative to the sequence's first query, clamped so the window
   // test is one unsigned compare; an empty slot and a query past n are
   // outside every window.
   constexpr int32_t kFar = 1 << 30;
   int32_t crel[QB];
-  // fp32: dims 16g .. 16g+15; bf16: dims 32c + 8g .. +7 for c = 0, 1
-  float qv[QB][16];
 #pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    const int r = qb * 16 + qc;
-    crel[qb] = r < n ? r : -kFar;
-#pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      const int dim = KV_BF16 ? (i >> 3) * 32 + g * 8 + (i & 7) : g * 16 + i;
-      const float4 t = r < n ? *(const float4*)&q_l[r][dim] : make_float4(0.f, 0.f, 0.f, 0.f);
-      qv[qb][i] = t.x; qv[qb][i + 1] = t.y; qv[qb][i + 2] = t.z; qv[qb][i + 3] = t.w;
-    }
-  }
-  bf16x8_t qh[QB][2], ql[QB][2];
-  if constexpr (KV_BF16) {
+  for (int qb = 0; qb < QB; qb++) crel[qb] = qb * 16 + qc < n ? qb * 16 + qc : -kFar;
+  float qv[QB][16];  // fp32 rings: dims 16g .. 16g + 15 of query qb * 16 + qc
+  if constexpr (!KV_BF16) {
 #pragma unroll
     for (int qb = 0; qb < QB; qb++)
 #pragma unroll
-      for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const float x = qv[qb][c * 8 + e];
-          const __bf16 hi = (__bf16)x;
-          qh[qb][c][e] = hi;
-          ql[qb][c][e] = (__bf16)(x - (float)hi);
-        }
+      for (int i = 0; i < 16; i += 4) {
+        const float4 t = *(const float4*)&q_l[qb * 16 + qc][g * 16 + i];
+        qv[qb][i] = t.x; qv[qb][i + 1] = t.y; qv[qb][i + 2] = t.z; qv[qb][i + 3] = t.w;
+      }
   }
   f32x4_t acc[QB][4];
 #pragma unroll
@@ -963,8 +963,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
     l[qb] = 0.f;
   }
 
-  for (int gi = g0; gi < groups; gi += step) {
-    load_group(gi + step < groups ? gi + step : gi, nxt);  // past the wave's last group: a reload, unused
+  auto compute = [&](int gi) {
     const int s0 = gi * 16;
     float kf[16];
     bf16x8_t kh[2];
@@ -1015,8 +1014,9 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
       if constexpr (KV_BF16) {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-          sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[c], qh[qb][c], sc, 0, 0, 0);
-          sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[c], ql[qb][c], sc, 0, 0, 0);
+          const int e = swz(qb * 16 + qc, c * 4 + g);  // dims 32c + 8g .. + 7
+          sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[c], *(const bf16x8_t*)&q_p[0][e], sc, 0, 0, 0);
+          sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[c], *(const bf16x8_t*)&q_p[1][e], sc, 0, 0, 0);
         }
       } else {
 #pragma unroll
@@ -1070,7 +1070,22 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
             acc[qb][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j][d], pw[j], acc[qb][d], 0, 0, 0);
       }
     }
-    cur = nxt;
+  };
+  // The last group has no load after it: reloading a group there to keep one
+  // loop body was 1 load in 5 at a window of 500 slots.  With q's parts in
+  // LDS, four frames, bf16 rings: 32 / 100 / 256 voices 2443 -> 2430, 4605 ->
+  // 4513, 8749 -> 8560 us; fp32 rings 32 / 256 voices 3287 -> 3267, 14702 ->
+  // 14638.
+  if (g0 < groups) {
+    int gi = g0;
+    for (; gi + step < groups; gi += step) {
+      load_group(gi + step, nxt);
+      if constexpr (KV_BF16)
+        asm volatile("" ::: "memory");  // q's parts are read again below, not kept in registers
+      compute(gi);
+      cur = nxt;
+    }
+    compute(gi);
   }
 
   // fold the waves: lane (qc, g) holds dims 4((g*4) + r) + d of query qb*16 + qc
