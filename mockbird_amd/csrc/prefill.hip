@@ -751,7 +751,7 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
 // every query of the chunk against its groups, reading K and V straight from
 // HBM into MFMA operands (no LDS staging).  A wave's first group is issued
 // before the chunk's rows are written when it holds none of their slots
-// (else after), and is in flight while its q rows are loaded and split
+// (else after), and is in flight while the rows are written
 // (64 voices 1.158 -> 1.150 ms per codec frame, 256 voices level).  Scores
 // are S^T[16 slots][16 queries]; the P V output block
 // d holds dims 4i + d in row i, so in the step for slot 4g + j (g = lane/16)
@@ -782,7 +782,18 @@ constexpr int kWindowSplitBlocks = 256;  // workgroups of a split launch at most
 constexpr int WPART = HD + 4;  // floats of a SPLIT state: 64 sums, max (log2 units), denominator
 static_assert((size_t)kWindowSplitBlocks * 32 * WPART <= kWindowPartFloats, "split states");
 
-template <bool KV_BF16, int QB, int NW, bool SPLIT>
+// K and V loads, with the streaming hint if ST.  An fp32 ring's K keeps plain
+// loads: a lane reads its 64 bytes of a row in four instructions, and with the
+// hint the lines do not stay for the later ones (200 voices, four frames 13.50
+// -> 14.91 ms; V alone, whole lines per instruction, 13.15).
+template <bool ST, class T>
+__device__ __forceinline__ T load_kv(const char* p) {
+  typedef uint32_t Vec __attribute__((ext_vector_type(sizeof(T) / 4)));
+  if constexpr (ST) return __builtin_bit_cast(T, __builtin_nontemporal_load((const Vec*)p));
+  else return *(const T*)p;
+}
+
+template <bool KV_BF16, int QB, int NW, bool SPLIT, bool ST>
 __global__ __launch_bounds__(64 * NW) void k_attn_window(
     const float* __restrict__ qkv, Rows qkv_rows, const int32_t* __restrict__ pos0,
     const int32_t* __restrict__ n_rows, void* __restrict__ ring_k, void* __restrict__ ring_v,
@@ -829,7 +840,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
     const int ks = min(s0 + qc, kv_end - 1);
     if constexpr (KV_BF16) {
 #pragma unroll
-      for (int c = 0; c < 2; c++) r.k[c] = *(const uint4*)(kb + ((int64_t)ks * HD + c * 32 + g * 8) * 2);
+      for (int c = 0; c < 2; c++) r.k[c] = load_kv<ST, uint4>(kb + ((int64_t)ks * HD + c * 32 + g * 8) * 2);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; i++) r.k[i] = *(const uint4*)(kb + ((int64_t)ks * HD + g * 16 + 4 * i) * 4);
@@ -839,11 +850,11 @@ __global__ __launch_bounds__(64 * NW) void k_attn_window(
       const int sl = s0 + 4 * g + j;
       const int vs = min(sl, kv_end - 1);
       if constexpr (KV_BF16) {
-        const uint2 w = *(const uint2*)(vb + ((int64_t)vs * HD + 4 * qc) * 2);
+        const uint2 w = load_kv<ST, uint2>(vb + ((int64_t)vs * HD + 4 * qc) * 2);
         if (j & 1) { r.v[j >> 1].z = w.x; r.v[j >> 1].w = w.y; }
         else { r.v[j >> 1].x = w.x; r.v[j >> 1].y = w.y; }
       } else {
-        r.v[j] = *(const uint4*)(vb + ((int64_t)vs * HD + 4 * qc) * 4);
+        r.v[j] = load_kv<ST, uint4>(vb + ((int64_t)vs * HD + 4 * qc) * 4);
       }
       r.p[j] = sp[vs];
     }
@@ -1199,10 +1210,18 @@ int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_m
   constexpr int NW = kWindowWaves;
   const int S = part ? window_splits(ring.heads * B, ring.C) : 1;
   const dim3 grid((unsigned)ring.heads, (unsigned)B, (unsigned)S);
-  auto go = [&](auto bf_, auto qb_, auto split_) {
-    constexpr bool BF = decltype(bf_)::value, SP = decltype(split_)::value;
+  // A window is read once a frame.  Once all layers' rings exceed the last-level
+  // cache (24 MB a voice in bf16, 48 in fp32) loads with the streaming hint are
+  // the faster ones; below that they lose what the cache keeps until the next
+  // frame.  Four frames, plain -> hint: bf16 4 / 8 / 16 / 32 / 64 / 256 voices
+  // 1554 -> 1572, 1630 -> 1620, 1997 -> 1806, 2431 -> 2225, 3263 -> 3037, 8391 ->
+  // 8185 us; fp32 1 / 4 / 8 / 12 / 64 / 200 voices 1754 -> 1769, 1818 -> 1820,
+  // 2206 -> 1955, 2446 -> 2317, 4753 -> 4618, 13564 -> 13153.
+  const bool stream = ring.heads * B * (ring.bf16 ? 2 : 4) >= 64;
+  auto go = [&](auto bf_, auto qb_, auto split_, auto st_) {
+    constexpr bool BF = decltype(bf_)::value, SP = decltype(split_)::value, ST = decltype(st_)::value;
     constexpr int QB = decltype(qb_)::value;
-    hipLaunchKernelGGL((k_attn_window<BF, QB, NW, SP>), grid, dim3(64 * NW), 0, ctx->stream, qkv,
+    hipLaunchKernelGGL((k_attn_window<BF, QB, NW, SP, ST>), grid, dim3(64 * NW), 0, ctx->stream, qkv,
                        qkv_rows, pos0, n_rows, ring.k, ring.v, ring.sp, ring.seq_stride, ring.C,
                        ring.window, ring.wrap, ctx->rope_tab, out, out_rows, part);
   };
@@ -1214,13 +1233,16 @@ int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_m
   };
   using std::integral_constant;
   auto all = [&](auto qb_) {
-    if (S == 1) {
-      if (ring.bf16) go(std::true_type{}, qb_, std::false_type{});
-      else go(std::false_type{}, qb_, std::false_type{});
-      return;
-    }
-    if (ring.bf16) go(std::true_type{}, qb_, std::true_type{});
-    else go(std::false_type{}, qb_, std::true_type{});
+    auto by_type = [&](auto split_) {
+      auto by_hint = [&](auto bf_) {
+        if (stream) go(bf_, qb_, split_, std::true_type{});
+        else go(bf_, qb_, split_, std::false_type{});
+      };
+      if (ring.bf16) by_hint(std::true_type{});
+      else by_hint(std::false_type{});
+    };
+    if (S == 1) return by_type(std::false_type{});
+    by_type(std::true_type{});
     if (S == 2) merge(qb_, integral_constant<int, 2>{});
     else if (S == 4) merge(qb_, integral_constant<int, 4>{});
     else if (S == 8) merge(qb_, integral_constant<int, 8>{});

@@ -160,12 +160,14 @@ def test_codec_full_size_long_run(B, kv, frames):
     say(f"  max error / scale over {len(watch)} voices: {worst:.2e}")
 
 
-@pytest.mark.parametrize("B,kv", [(1, mb.MB_KV_F32), (3, mb.MB_KV_BF16), (17, mb.MB_KV_F32)])
+@pytest.mark.parametrize("B,kv", [(1, mb.MB_KV_F32), (3, mb.MB_KV_BF16), (9, mb.MB_KV_BF16),
+                                  (17, mb.MB_KV_F32)])
 def test_codec_shared_windows(B, kv):
     """Few voices: each (voice, head) window is shared between workgroups and
     merged.  Windows just past 2, 2, 4 and 8 workgroups' worth of 16-slot
     groups (8 waves each), decoded from empty rings (workgroups without a
-    group) until stages 2-4 wrap; 17 voices split the long windows only."""
+    group) until stages 2-4 wrap; 17 voices split the long windows only.
+    9 and 17 voices load the window with the streaming hint, 1 and 3 without."""
     say(f"codec shared windows, {B} voices, kv={kv}")
     layers, context = (1, 1, 1, 1), (245, 260, 520, 1030)
     watch = sorted({0, B // 2, B - 1})
