@@ -204,9 +204,10 @@ int mb_append_attend_dev(mb_ctx* ctx, int layer, int B, const void* qkv, int qkv
  * bias may be NULL; epi MB_EPI_STORE writes, MB_EPI_GELU applies gelu-tanh,
  * MB_EPI_ADD adds into C (the residual), MB_EPI_GELU_ERF applies the exact
  * (erf) GELU, and MB_EPI_SCALE_ADD reads `bias` as a per-column scale s and
- * stores C + s * (A W) (the codec's layer scale).  fp32 products and
- * accumulation.  Needs N % 64 == 0, K % 64 == 0, lda and ldc multiples of 4
- * and 16-byte aligned pointers.  Replaces GEMM_NT (kernels-batch.ts:156-184,
+ * stores C + s * (A W) (the codec's layer scale).  fp32 accumulation of fp32
+ * products, or of bf16 plane products that stand for them to 2^-24.  Needs
+ * N % 64 == 0, K % 64 == 0, lda and ldc multiples of 4 and 16-byte aligned
+ * pointers.  Replaces GEMM_NT (kernels-batch.ts:156-184,
  * called prefill.ts:404-422, :464-482), GEMV / GEMV_NOB (kernels-decode.ts:
  * 127-166, called decode.ts:517-526, :553-562, codec.ts:536-735) with the
  * GELU_TANH / GELU_ERF / ADD_RESIDUAL / LAYER_SCALE_ADD passes that follow
