@@ -783,15 +783,17 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ p
 }
 
 // Whether a streaming launch multiplies bf16 planes (k_gemm_stream's PLANES):
-// 48- and 64-row tiles, and 32-row tiles over at least 512 k.  There the fp32
+// tiles of 32 rows and more over at least 512 k.  There the fp32
 // matrix rate bounds the loop; smaller tiles wait for W, and the splits only
 // add to that.  fp32 MFMA -> planes, us: 2304 x 768 at 281 / 500 / 1000 rows
 // 12.3 -> 10.7, 34.4 -> 24.7, 57.7 -> 36.8 (48- and 64-row tiles); 768 x 3072
 // at 100 / 281 / 1000 rows 11.3 -> 10.9, 17.5 -> 15.8, 39.6 -> 31.5 (32-row
 // ones); 256 x 256 at 2048 rows 4.9 -> 5.2, 768 x 768 at 64 rows 5.5 -> 6.1
-// (16-row tiles).
+// (16-row tiles).  Over 256 k a wave has two blocks to split for: four
+// codec frames of 40 / 64 / 100 voices took 4087 / 4601 / 7348 us with planes in
+// the 48- and 64-row tiles, 4015 / 4512 / 7296 with fp32 products.
 static bool stream_planes(int mt, int K, int kw) {
-  return kw % (2 * kStreamChunk) == 0 && (mt >= 48 || (mt == 32 && K >= 512));
+  return kw % (2 * kStreamChunk) == 0 && (mt >= 32 && K >= 512);
 }
 
 // part_ext (optional, part_cap floats) holds the split-K partials instead of
