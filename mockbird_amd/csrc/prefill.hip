@@ -588,7 +588,9 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
     }
     if (tid < KS) Ps[bb][tid] = rp;
   };
-  load(0);
+  // every position of the tile's rows negative (kv_end <= 0): no slot is read,
+  // and the rows are zero
+  if (kv_end > 0) load(0);
 
   // B operands of the score MFMA: the planes of Q[row][32 kc + 8 grp + 0..7]
   // times 1/sqrt(64) * log2(e) (one fp32 rounding), so the MFMAs yield the
@@ -702,7 +704,7 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
     }
   };
 
-  stash(0);
+  if (kv_end > 0) stash(0);
   if (KS < kv_end) load(KS);
   int bb = 0;
   for (int t0 = 0; t0 < kv_end; t0 += KS) {

@@ -88,6 +88,44 @@ def test_prefill_fp32_tile_edges(kv, C):
                 assert err < 2e-5, (past, b, err)
 
 
+@pytest.mark.parametrize("kv", [mb.MB_KV_F32, mb.MB_KV_BF16])
+def test_prefill_fp32_negative_positions(kv):
+    """Device positions are not checked: a row at a negative one sees no slot
+    and comes out zero, whole tiles of them (the first sequence, whose rings
+    start the allocation) read nothing, and the rows from position 0 on are
+    the oracle's.  Bar: test_prefill_fp32_tile_edges'."""
+    torch = pytest.importorskip("torch")
+    say(f"prefill fp32 negative positions kv={kv}")
+    B, R, C = 3, 100, 64
+    dev = torch.device("cuda")
+    pos0 = np.array([-1000, -70, -3], np.int32)
+    n = np.array([R, R, 40], np.int32)
+    with mb.Context(n_layers=1, capacity=C, max_seqs=B, max_rows=R, kv_dtype=kv) as ctx:
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        ring = oracle.Ring(B, C, kv_bf16=(kv == mb.MB_KV_BF16))
+        zero = np.zeros(B, np.int32)
+        first = synth.qkv_rows(81, (B, 50))
+        ctx.ring_write_rows(0, first, zero, zero + 50)
+        ring.write(first, zero, zero + 50)
+        q = synth.qkv_rows(82, (B, R))[..., :768].copy()
+        tq = torch.from_numpy(q).to(dev)
+        p0, tn = torch.from_numpy(pos0).to(dev), torch.from_numpy(n).to(dev)
+        out = torch.full((B, R, 768), 7.0, device=dev)
+        ctx.prefill_attention_dev(0, B, R, tq.data_ptr(), p0.data_ptr(), tn.data_ptr(), out.data_ptr())
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        for b in range(B):
+            neg = min(-int(pos0[b]), int(n[b]))
+            assert not got[b, :neg].any(), b
+            assert (got[b, n[b]:] == 7.0).all(), b
+            if neg < n[b]:
+                qb = np.zeros((B, n[b] - neg, 768), np.float32)
+                qb[b] = q[b, neg:n[b]]
+                want = ring.attend_prefill(qb, zero, zero + (n[b] - neg))[b]
+                err = np.abs(got[b, neg:n[b]] - want).max()
+                assert err < 2e-5, (b, err)
+
+
 def test_prefill_rows_are_independent():
     """A sequence cut to its first 300 rows gets bit-identical outputs for
     those rows (the causal-prefix property of the reference captures)."""
