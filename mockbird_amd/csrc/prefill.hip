@@ -163,6 +163,13 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
   const int rlast = min(qtile * BQ + BQ, n) - 1;
   const int64_t kv_end64 = p0 + rlast + 1;
   const int kv_end = kv_end64 < C ? (int)kv_end64 : C;
+  if (kv_end <= 0) {  // every position negative: no slot to read, rows of zeros
+    const int first = qtile * BQ;
+    for (int i = tid; i < (rlast + 1 - first) * (HD / 4); i += 64 * NW)
+      *(f32x4_t*)(out + row_at(out_rows, b, first + i / (HD / 4)) + h * HD + i % (HD / 4) * 4) =
+          f32x4_t{0.f, 0.f, 0.f, 0.f};
+    return;  // uniform per workgroup, before any barrier
+  }
 
   // B operands of the score MFMA: Q[row][32*kc + 8*grp + 0..7] times
   // 1/sqrt(64) * log2(e), rounded to bf16 once here, so the MFMA yields the
@@ -425,7 +432,7 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
     }
   };
   // the first tile and q, then every later tile two tiles ahead of its use
-  // (kv_end >= 1: the workgroup has rows)
+  // (kv_end >= 1 here)
   using std::integral_constant;
   issue(0, 0);
   MB_WAIT_VMCNT(0);

@@ -88,17 +88,18 @@ def test_prefill_fp32_tile_edges(kv, C):
                 assert err < 2e-5, (past, b, err)
 
 
-@pytest.mark.parametrize("kv", [mb.MB_KV_F32, mb.MB_KV_BF16])
-def test_prefill_fp32_negative_positions(kv):
+@pytest.mark.parametrize("kv,bf16_q", [(mb.MB_KV_F32, False), (mb.MB_KV_BF16, False),
+                                       (mb.MB_KV_BF16, True)])
+def test_prefill_negative_positions(kv, bf16_q):
     """Device positions are not checked: a row at a negative one sees no slot
     and comes out zero, whole tiles of them (the first sequence, whose rings
     start the allocation) read nothing, and the rows from position 0 on are
-    the oracle's.  Bar: test_prefill_fp32_tile_edges'."""
+    the oracle's.  Bars: test_prefill_fp32_tile_edges'; bf16 queries 2e-2."""
     torch = pytest.importorskip("torch")
-    say(f"prefill fp32 negative positions kv={kv}")
-    B, R, C = 3, 100, 64
+    say(f"prefill negative positions kv={kv} bf16 q={bf16_q}")
+    B, R, C = 3, 200, 64
     dev = torch.device("cuda")
-    pos0 = np.array([-1000, -70, -3], np.int32)
+    pos0 = np.array([-1000, -140, -3], np.int32)
     n = np.array([R, R, 40], np.int32)
     with mb.Context(n_layers=1, capacity=C, max_seqs=B, max_rows=R, kv_dtype=kv) as ctx:
         ctx.set_stream(torch.cuda.current_stream().cuda_stream)
@@ -108,10 +109,14 @@ def test_prefill_fp32_negative_positions(kv):
         ctx.ring_write_rows(0, first, zero, zero + 50)
         ring.write(first, zero, zero + 50)
         q = synth.qkv_rows(82, (B, R))[..., :768].copy()
+        if bf16_q:
+            q = oracle.bf16_round(q)
         tq = torch.from_numpy(q).to(dev)
+        tq = tq.to(torch.bfloat16) if bf16_q else tq
         p0, tn = torch.from_numpy(pos0).to(dev), torch.from_numpy(n).to(dev)
         out = torch.full((B, R, 768), 7.0, device=dev)
-        ctx.prefill_attention_dev(0, B, R, tq.data_ptr(), p0.data_ptr(), tn.data_ptr(), out.data_ptr())
+        ctx.prefill_attention_dev(0, B, R, tq.data_ptr(), p0.data_ptr(), tn.data_ptr(), out.data_ptr(),
+                                  q_dtype=mb.MB_DT_BF16 if bf16_q else mb.MB_DT_F32)
         torch.cuda.synchronize()
         got = out.cpu().numpy()
         for b in range(B):
@@ -123,7 +128,7 @@ def test_prefill_fp32_negative_positions(kv):
                 qb[b] = q[b, neg:n[b]]
                 want = ring.attend_prefill(qb, zero, zero + (n[b] - neg))[b]
                 err = np.abs(got[b, neg:n[b]] - want).max()
-                assert err < 2e-5, (b, err)
+                assert err < (2e-2 if bf16_q else 2e-5), (b, err)
 
 
 def test_prefill_rows_are_independent():
