@@ -725,7 +725,55 @@ __global__ __launch_bounds__(256, 3) void k_flash_x(
       if (t0 + 2 * KS < kv_end) load(t0 + 2 * KS);
     }
   }
-  const float l = col_sum(lsum);
+  float l = col_sum(lsum);
+  // An infinity has no planes (inf - inf), and 0 times one in a plane is NaN.
+  // A wave with a sum that is not finite takes its rows again, slot by slot
+  // over the live slots with fp32 products: infinities and NaN reach the rows
+  // that see them, as those products give them, and no others.
+  float nf = lsum;
+#pragma unroll
+  for (int d = 0; d < 4; d++) nf += (acc[d][0] + acc[d][1]) + (acc[d][2] + acc[d][3]);
+  if (wave_rows && __ballot(!(fabsf(nf) < INFINITY))) {  // uniform
+    const float* src = q + row_at(q_rows, b, min(r, n - 1)) + h * HD + grp * 4;
+    f32x4_t qf[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+      qf[d] = *(const f32x4_t*)(src + 16 * d) * kScoreLog2;
+      acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    auto dims = [&](const char* base, int slot, int d) {  // dims 16d + 4 grp .. + 3
+      const int64_t e = (int64_t)slot * HD + 16 * d + 4 * grp;
+      if constexpr (KV_BF16) {
+        const uint2 w = *(const uint2*)(base + e * 2);
+        return f32x4_t{__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u),
+                       __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xffff0000u)};
+      } else {
+        return *(const f32x4_t*)(base + e * 4);
+      }
+    };
+    float m = -INFINITY;
+    l = 0.f;
+    for (int slot = 0; slot < kv_end; slot++) {
+      const int32_t ps = sp[slot];
+      const bool live = ps >= 0 && (uint32_t)(crel - (ps - ref)) < (uint32_t)W;
+      if (!__ballot(live)) continue;  // uniform
+      float x = 0.f;
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        const f32x4_t k = dims(kb, slot, d);
+        x += (qf[d][0] * k[0] + qf[d][1] * k[1]) + (qf[d][2] * k[2] + qf[d][3] * k[3]);
+      }
+      x = col_sum(x);
+      if (live) {
+        const float mn = fmaxf(m, x), mu = mn == -INFINITY ? 0.f : mn;
+        const float scale = __builtin_amdgcn_exp2f(m - mu), p = __builtin_amdgcn_exp2f(x - mu);
+        m = mn;
+        l = l * scale + p;
+#pragma unroll
+        for (int d = 0; d < 4; d++) acc[d] = acc[d] * scale + dims(vb, slot, d) * p;
+      }
+    }
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (r >= n) return;
   if constexpr (PO == 0) {

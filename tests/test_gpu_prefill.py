@@ -131,6 +131,64 @@ def test_prefill_negative_positions(kv, bf16_q):
                 assert err < (2e-2 if bf16_q else 2e-5), (b, err)
 
 
+@pytest.mark.parametrize("kv", [mb.MB_KV_F32, mb.MB_KV_BF16])
+def test_prefill_fp32_infinities_and_nan(kv):
+    """fp32 queries over a ring with infinities and NaN, against float64: an
+    infinite V reaches the rows that see its slot and leaves the others
+    finite, a slot whose score is -inf drops out, one at +inf and a NaN make
+    their rows NaN, and finite values above the largest bf16 stay what they
+    are.  Finite rows: test_prefill_fp32_tile_edges' bar, relative to the
+    largest |v|."""
+    torch = pytest.importorskip("torch")
+    say(f"prefill infinities kv={kv}")
+    B, R, C = 6, 90, 128
+    dev = torch.device("cuda")
+    g = np.random.default_rng(83)
+    x = g.standard_normal((B, R, 3, 12, 64)).astype(np.float32)
+    x[0, 20, 2, 3, 5], x[0, 60, 2, 3, 6] = np.inf, -np.inf   # V, either sign
+    x[0, 70, 2, 3, 5] = -np.inf                              # ... and both in one dim
+    x[1, 30, 1, :, 9] = np.inf                               # K: score -inf or +inf by q's sign
+    x[1, :, 0, 0, 9] = -np.abs(x[1, :, 0, 0, 9]) - 1         # head 0: always dropped
+    x[2, 40, 2, 7, 11], x[2, 50, 1, 8, 12] = np.nan, np.nan
+    x[3, 44, 0, 2, 1] = np.inf                               # q
+    x[4, 10, 2, 5, 8] = 1e30                                 # large, finite
+    if kv == mb.MB_KV_F32:
+        x[5, 0, 2, 4, 3] = 3.4e38                            # above the largest bf16
+    if kv == mb.MB_KV_BF16:
+        x[:, :, 1:] = oracle.bf16_round(x[:, :, 1:])
+    q, k, v = (np.ascontiguousarray(x[:, :, i].reshape(B, R, 768)) for i in range(3))
+    with mb.Context(n_layers=1, capacity=C, max_seqs=B, max_rows=R, kv_dtype=kv) as ctx:
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        pos = np.arange(R, dtype=np.int32)
+        for b in range(B):
+            ctx.write_ring(0, b, 0, k[b], v[b], pos)
+        tq = torch.from_numpy(q).to(dev)
+        p0 = torch.zeros(B, dtype=torch.int32, device=dev)
+        n = torch.full((B,), R, dtype=torch.int32, device=dev)
+        out = torch.empty((B, R, 768), device=dev)
+        ctx.prefill_attention_dev(0, B, R, tq.data_ptr(), p0.data_ptr(), n.data_ptr(), out.data_ptr())
+        torch.cuda.synchronize()
+        got = out.cpu().numpy().reshape(B, R, 12, 64)
+    with np.errstate(invalid="ignore"):
+        y = x.astype(np.float64)
+        for b in range(B):
+            for r in range(R):
+                for h in range(12):
+                    s = (y[b, r, 0, h] * y[b, :r + 1, 1, h]).sum(-1) / 8
+                    top = s.max()  # NaN if any is
+                    p = np.exp(s - top)
+                    want = (p[:, None] * y[b, :r + 1, 2, h]).sum(0) / p.sum()
+                    have = got[b, r, h].astype(np.float64)
+                    at = (b, r, h)
+                    assert np.array_equal(np.isnan(have), np.isnan(want)), at
+                    assert np.array_equal(np.isposinf(have), np.isposinf(want)), at
+                    assert np.array_equal(np.isneginf(have), np.isneginf(want)), at
+                    fin = np.isfinite(want)
+                    big = max(5.0, float(np.abs(np.where(np.isfinite(y[b, :r + 1, 2, h]),
+                                                         y[b, :r + 1, 2, h], 0)).max()))
+                    assert (np.abs(have - want)[fin] < 2e-5 / 5 * big).all(), at
+
+
 def test_prefill_rows_are_independent():
     """A sequence cut to its first 300 rows gets bit-identical outputs for
     those rows (the causal-prefix property of the reference captures)."""
