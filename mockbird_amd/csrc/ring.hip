@@ -576,6 +576,14 @@ __global__ __launch_bounds__(64 * MAXNW, !KV_BF16 && APPEND ? 3 : 1) void k_attn
     for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
 #pragma unroll
     for (int s = 0; s < kSplitMaxWaves; s++) o = fmaf(__shfl(w, s), v[s], o);
+    // 0 times the last state is NaN where that is infinite: without the reread
+    // ones then (left out from the start: 88.4 -> 91.0 us, 12 layers of a voice)
+    if (__ballot(!(fabsf(o) < INFINITY))) {  // uniform
+      o = 0.f;
+#pragma unroll
+      for (int s = 0; s < kSplitMaxWaves; s++)
+        if (s < nwp) o = fmaf(__shfl(w, s), v[s], o);
+    }
     out[row_at(out_rows, b, r) + head * HD + lane] = L > 0.f ? o / L : 0.f;
     if (lane == 0) __hip_atomic_store(&ws.count[unit], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;

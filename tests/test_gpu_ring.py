@@ -438,6 +438,32 @@ def test_units_shared_between_waves(name, kv, B, C):
     assert np.abs(got[0, :, :768] - want).max() < (2e-6 if kv == mb.MB_KV_F32 else 1e-4)
 
 
+@pytest.mark.parametrize("name,kv", KV)
+def test_shared_unit_keeps_an_infinite_value(name, kv):
+    """A unit shared by fewer waves than the most there can be, an infinite V
+    in the last one's batch: its dim comes out infinite, the others as the
+    oracle's without it (1e-4)."""
+    say(f"shared unit, infinite V kv={name}")
+    C, pos = 1000, np.array([700], np.int32)  # 11 or 15 batches of at most 64 slots
+    rng = np.random.default_rng(91)
+    k, v = (rng.standard_normal((701, 768)).astype(np.float32) for _ in range(2))
+    if kv == mb.MB_KV_BF16:
+        k, v = oracle.bf16_round(k), oracle.bf16_round(v)
+    q = rng.standard_normal((1, 768)).astype(np.float32)
+    bad = v.copy()
+    bad[690, 5 * 64 + 7], bad[690, 11 * 64 + 63] = np.inf, -np.inf
+    with mb.Context(n_layers=1, capacity=C, max_seqs=1, max_rows=1, kv_dtype=kv) as ctx:
+        ctx.write_ring(0, 0, 0, k, v, np.arange(701, dtype=np.int32))
+        want = ctx.decode_attention(0, q, pos)[0]
+        ctx.write_ring(0, 0, 0, k, bad, np.arange(701, dtype=np.int32))
+        got = ctx.decode_attention(0, q, pos)[0]
+    ring = _oracle_ring(1, C, kv)
+    ring.K[0, :701], ring.V[0, :701], ring.slot_pos[0, :701] = k, v, np.arange(701)
+    assert np.abs(want - ring.attend(q, pos)[0]).max() < 1e-4
+    want[5 * 64 + 7], want[11 * 64 + 63] = np.inf, -np.inf
+    assert np.array_equal(got, want)
+
+
 def test_append_attend_range_error_on_a_non_wrapping_ring():
     say("fused append+attention range error")
     import torch
