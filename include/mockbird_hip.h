@@ -205,7 +205,8 @@ int mb_append_attend_dev(mb_ctx* ctx, int layer, int B, const void* qkv, int qkv
  * MB_EPI_ADD adds into C (the residual), MB_EPI_GELU_ERF applies the exact
  * (erf) GELU, and MB_EPI_SCALE_ADD reads `bias` as a per-column scale s and
  * stores C + s * (A W) (the codec's layer scale).  fp32 accumulation of fp32
- * products, or of bf16 plane products that stand for them to 2^-24.  Needs
+ * products, or of sums of bf16 plane products that leave out at most 2^-24 of
+ * each (and hand infinities and NaN on as fp32 products do).  Needs
  * N % 64 == 0, K % 64 == 0, lda and ldc multiples of 4 and 16-byte aligned
  * pointers.  Replaces GEMM_NT (kernels-batch.ts:156-184,
  * called prefill.ts:404-422, :464-482), GEMV / GEMV_NOB (kernels-decode.ts:

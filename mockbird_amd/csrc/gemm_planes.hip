@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void k_split_w3(const float* __restrict__ Wt, 
   float v[8];
 #pragma unroll
   for (int t = 0; t < 8; t++) v[t] = src[t * 64];
-  const Planes w = split3(v);
+  const Planes w = split3<true>(v);
 #pragma unroll
   for (int p = 0; p < 3; p++) Wx[(blk * 4 + j) * 192 + p * 64 + lane] = __builtin_bit_cast(uint4, w.p[p]);
 }

@@ -402,7 +402,7 @@ int launch_gemm_x3(mb_ctx* ctx, int epi, const float* A, int64_t lda, const void
 // if not null) of 768-wide rows, and
 // launch_gemm_planes computes epi(A W + lnd + bias) from pa planes of A and pw
 // of W (2 x 2: the products of launch_gemm_x3, on its weight copies; 2 x 1:
-// launch_gemm_x2's; 3 x 3: fp32 products to 2^-24, on launch_split_w3's copies
+// launch_gemm_x2's; 3 x 3: all but 2^-24 of each fp32 product, on launch_split_w3's copies
 // of a column-block-major W, 6 K N bytes).  out_planes (GELU epilogues): the result goes there as
 // the planes of the next projection's operand, not to Cm.  N a multiple of
 // 128, K of 32.

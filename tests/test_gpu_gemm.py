@@ -71,10 +71,12 @@ PLANE_SHAPES = [  # (M, N, K): 32-, 48- and 64-row tiles of the streaming kernel
 @pytest.mark.parametrize("M,N,K", PLANE_SHAPES)
 def test_linear_planes_hold_fp32(ctx, M, N, K):
     """Products of three bf16 planes stand for fp32 ones: each is within
-    3 2^-24 of |a w| (the plane pairs left out) and the fp32 sums round at
-    most K / 128 times per wave beyond that, so an output is within
-    8 2^-24 sum |a w| of float64 -- operands over 30 binary orders, where a
-    two-plane split is off by 2^-16."""
+    2^-24 (1 + 2^-9) of |a w| (the plane pairs left out,
+    test_linear_plane_products_one_by_one).  The fp32 sums round six times per
+    32 k of a wave's share: 36 to 144 times 2^-24 if all went one way at full
+    size, a few times it as they fall.  An output is held to 8 2^-24 sum |a w|
+    of float64 -- operands over 30 binary orders, where a two-plane split is
+    off by 2^-16."""
     torch = pytest.importorskip("torch")
     say(f"linear planes M={M} N={N} K={K}")
     g = np.random.default_rng([M, N, K, 1])
@@ -91,6 +93,40 @@ def test_linear_planes_hold_fp32(ctx, M, N, K):
     worst = float(((tC.double() - want).abs() / size).max()) * 2 ** 24
     say(f"  worst error {worst:.2f} x 2^-24 sum |a w|")
     assert worst < 8
+
+
+@pytest.mark.parametrize("M,N,K", [(281, 2304, 768), (100, 768, 3072), (600, 768, 512)])
+def test_linear_plane_products_one_by_one(ctx, M, N, K):
+    """One nonzero value in each row of A, so that every output is one product
+    and shows what the plane pairs left out take from it: at most 2^-24 (1 +
+    2^-9).  The six kept pairs are added by the matrix unit, whose sums are
+    within an ulp, not half of one (against sums rounded to nearest 16 % of
+    these outputs are the next float): 2^-23 once at full size and five times
+    at 2^-8 of it, 3.1 2^-24 with the pairs left out.  Mantissas where planes
+    cut (7.8 2^-24) or rounded lose most, and random ones."""
+    torch = pytest.importorskip("torch")
+    say(f"linear plane products M={M} N={N} K={K}")
+    g = np.random.default_rng([M, N, K, 2])
+
+    def values(*shape):
+        hard = np.array([0x00FFFF, 0x00FEFF, 0x007FC0, 0x008040, 0x007FFF, 0x7FFFFF, 0], np.uint32)
+        mant = np.where(g.random(shape) < 0.5, g.choice(hard, shape), g.integers(0, 1 << 23, shape))
+        bits = mant.astype(np.uint32) | (g.integers(97, 158, shape).astype(np.uint32) << 23)
+        return (bits | (g.integers(0, 2, shape).astype(np.uint32) << 31)).view(np.float32)
+
+    A = np.zeros((M, K), np.float32)
+    A[np.arange(M), g.integers(0, K, M)] = values(M)
+    W = values(K, N)
+    dev = torch.device("cuda")
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    tA, tW = torch.from_numpy(A).to(dev), torch.from_numpy(W).to(dev)
+    tC = torch.zeros((M, N), device=dev)
+    ctx.linear_dev(M, N, K, tA.data_ptr(), K, tW.data_ptr(), None, tC.data_ptr(), N)
+    torch.cuda.synchronize()
+    want = tA.double() @ tW.double()
+    worst = float(((tC.double() - want) / want).abs().max()) * 2 ** 24
+    say(f"  worst error {worst:.2f} x 2^-24 |a w|")
+    assert worst < 3.1
 
 
 def test_linear_planes_keep_infinities_and_nan(ctx):

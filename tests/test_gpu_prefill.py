@@ -63,8 +63,8 @@ def test_prefill_continuation_over_a_wrapped_ring():
 def test_prefill_fp32_tile_edges(kv, C):
     """Row counts around a wave's 16 queries, a workgroup's 64 and the 32- and
     64-slot tiles, after 0 / 31 / 90 earlier rows (rings of 100 slots wrap).
-    Bar: a score is 64 products, each within 3 2^-24 of |q k| (the plane pairs
-    left out) and summed with 2^-24 roundings; at |q . k| / 8 < 8 a weight is
+    Bar: a score is 64 products, each within 2^-24 (1 + 2^-9) of |q k| (the
+    plane pairs left out) and summed to an ulp; at |q . k| / 8 < 8 a weight is
     within 1e-5, and so is the weighted mean of |v| < 5 to 2e-5 in the mean."""
     say(f"prefill fp32 tile edges kv={kv} C={C}")
     n = np.array([1, 15, 16, 17, 31, 33, 63, 64, 65, 96], np.int32)
