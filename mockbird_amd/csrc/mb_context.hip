@@ -91,7 +91,7 @@ static AttnSplit claim_split(mb_ctx* ctx) {
   }
   ctx->split_claimed = true;
   ctx->split_stream = ctx->stream;
-  return {ctx->split_part, ctx->split_count};
+  return {ctx->split_part[1], ctx->split_count[1]};
 }
 // After the context's stream has been synchronised.
 static void release_split(mb_ctx* ctx) {
@@ -239,13 +239,15 @@ int mb_create(const mb_config* cfg, mb_ctx** out) {
       e = hipMemcpy(ctx->rope_tab, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
       if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMemcpy(rope table)"); break; }
     }
-    e = hipMalloc(&ctx->split_part, kSplitFloats * 4 + kSplitMaxUnits * 4);
+    e = hipMalloc(&ctx->split_part[0], 2 * (kSplitFloats + kSplitMaxUnits) * 4);
     if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMalloc(attention split)"); break; }
-    ctx->split_count = (int32_t*)(ctx->split_part + kSplitFloats);
-    rc = launch_fill_i32(ctx, ctx->split_count, kSplitMaxUnits, 0);
+    ctx->split_part[1] = ctx->split_part[0] + kSplitFloats;
+    ctx->split_count[0] = (int32_t*)(ctx->split_part[1] + kSplitFloats);
+    ctx->split_count[1] = ctx->split_count[0] + kSplitMaxUnits;
+    rc = launch_fill_i32(ctx, ctx->split_count[0], 2 * kSplitMaxUnits, 0);
     if (rc) break;
     ctx->device_bytes = 2 * (int64_t)ctx->ring_bytes + slots * 4 + (int64_t)kRopeTab * 32 * 8 +
-                        (int64_t)(kSplitFloats + kSplitMaxUnits) * 4;
+                        (int64_t)2 * (kSplitFloats + kSplitMaxUnits) * 4;
     // every slot empty; K/V zero so a read of an unwritten slot is well defined
     rc = launch_fill_kv(ctx, ctx->ring_k, (int64_t)(ctx->ring_bytes / kv_elem_bytes(ctx)), 0.f);
     if (rc) break;
@@ -276,7 +278,7 @@ void mb_destroy(mb_ctx* ctx) {
   (void)hipFree(ctx->ring_v);
   (void)hipFree(ctx->slot_pos);
   (void)hipFree(ctx->rope_tab);
-  (void)hipFree(ctx->split_part);
+  (void)hipFree(ctx->split_part[0]);
   for (void* p : {(void*)ctx->local_k, (void*)ctx->local_v, (void*)ctx->local_sp,
                   (void*)ctx->local_pos, (void*)ctx->seen, (void*)ctx->tokens, (void*)ctx->cont})
     (void)hipFree(p);

@@ -133,11 +133,13 @@ struct mb_ctx {
   int32_t* slot_pos = nullptr;
   size_t ring_bytes = 0;  // bytes of ring_k (== ring_v)
 
-  // The kernel-level attention calls' AttnSplit (mb_create).  It is used by
-  // one stream at a time: the first call after the last synchronising one
-  // claims it (claim_split), calls on other streams run without.
-  float* split_part = nullptr;
-  int32_t* split_count = nullptr;
+  // The AttnSplits (mb_create), first the model's steps', which like their
+  // activations serve one call at a time, then the kernel-level attention
+  // calls'.  The second is used by one stream at a time: the first call after
+  // the last synchronising one claims it (claim_split), calls on other
+  // streams run without.
+  float* split_part[2] = {};
+  int32_t* split_count[2] = {};
   bool split_claimed = false;
   hipStream_t split_stream = nullptr;
 

@@ -296,16 +296,6 @@ int run_layer_planes(mb_ctx* ctx, int P, const LayerW& w, const RingView& ring, 
   return launch_gemm_planes(ctx, P, pw, EPI_ADD, a.ffn, fc_out, D, FFN, nullptr, w.fc_out_b, a.x, D, M);
 }
 
-// The workspace of the decode attention of few sequences; none for more.
-int attn_split(mb_ctx* ctx, int B, AttnSplit& s) {
-  if (B * H > kSplitMaxUnits) return MB_OK;
-  const bool fresh = !ctx->scratch["attn_split"].ptr;
-  s.part = (float*)scratch(ctx, "attn_split", kSplitFloats * 4 + kSplitMaxUnits * 4);
-  if (!s.part) return fail(ctx, MB_ERR_NOMEM, "attention split");
-  s.count = (int32_t*)(s.part + kSplitFloats);
-  return fresh ? launch_fill_i32(ctx, s.count, kSplitMaxUnits, 0) : MB_OK;
-}
-
 // One d=768 layer over M rows held in a.x.  Rows belong to B sequences with
 // n_rows[b] rows at positions pos0[b] + r (packed by `packed` when prefill is
 // set, else one row per sequence).  With `pick` (one row) the QKV projection
@@ -347,12 +337,10 @@ int run_layer(mb_ctx* ctx, const LayerW& w, const RingView& ring, int B, int row
   // attention as per-wave partials merged by the O projection.
   const bool parts = !prefill && gemv && ctx->w_bf16 && pos_const < 0 && B <= kPartsMaxSeqs &&
                      ring.heads == H && ring.window == ring.C;
-  float* part = nullptr;
+  const AttnSplit split = {ctx->split_part[0], ctx->split_count[0]};
+  static_assert(kPartsMaxSeqs * H <= kSplitMaxUnits && kSplitMaxWaves >= 16, "partials");
+  float* const part = split.part;
   int nwp = 0;
-  if (parts) {
-    part = (float*)scratch(ctx, "attn_parts", (size_t)B * H * 16 * PART * sizeof(float));
-    if (!part) return fail(ctx, MB_ERR_NOMEM, "attention partials");
-  }
   Rows qkv_rows, q_rows;
   if (prefill) {
     qkv_rows.row_stride = QKV;
@@ -375,10 +363,8 @@ int run_layer(mb_ctx* ctx, const LayerW& w, const RingView& ring, int B, int row
     rc = launch_append_attn_parts(ctx, ring, B, a.qkv, pos0, max_valid, part, nwp);
   } else {
     // one launch appends this row's K/V and attends the ring including it
-    AttnSplit split;
-    if (pos_const < 0 && (rc = attn_split(ctx, B, split))) return rc;
     rc = launch_append_attn(ctx, ring, B, a.qkv, MB_DT_F32, qkv_rows, pos0, max_valid, nullptr,
-                            Rows{}, a.att, q_rows, pos_const, split);
+                            Rows{}, a.att, q_rows, pos_const, pos_const < 0 ? split : AttnSplit{});
   }
   if (rc) return rc;
   // decode sizes read the column-block-major copies of O and fc_out

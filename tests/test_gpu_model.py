@@ -514,6 +514,58 @@ def _per_call_frames(ctx, h, pos, max_pos, F, latch):
     return np.stack(out_codes), np.stack(out_cont)
 
 
+@pytest.mark.parametrize("kv", [mb.MB_KV_F32, mb.MB_KV_BF16])
+@pytest.mark.parametrize("storage", [mb.MB_W_F32, mb.MB_W_BF16])
+def test_few_voice_steps_in_a_callers_graph(kv, storage):
+    """A program that has run its many voices captures the step of a few:
+    nothing is allocated for it, eagerly or under capture, and every replay,
+    eager steps of other sizes between them, gives the eager step's bits."""
+    torch = pytest.importorskip("torch")
+    say(f"captured few-voice steps kv={kv} weights={storage}")
+    V, B, C, pos = 64, 64, 600, 450
+    g = np.random.default_rng(97)
+    w = synth.model_weights(n_layers=1, vocab=V, seed=7, bias_std=0.02, ln_std=0.1)
+    rows = torch.from_numpy(np.stack([synth.frame_row(g.integers(0, 1024, 16)) for _ in range(B)])
+                            .astype(np.int32)).cuda()
+    tpos = torch.full((B,), pos, dtype=torch.int32, device="cuda")
+    with _ctx(w, 1, V, B, C, kv) as ctx:
+        ctx.set_weight_storage(storage)
+        for b in range(16):
+            k, v = g.standard_normal((2, pos, 768), dtype=np.float32)
+            ctx.write_ring(0, b, 0, k, v, np.arange(pos, dtype=np.int32))
+        s = torch.cuda.Stream()
+        ctx.set_stream(s.cuda_stream)
+        many = torch.empty((B, 768), device="cuda")
+
+        def step(n, out):
+            ctx.decode_step_dev(n, rows.data_ptr(), tpos.data_ptr(), pos, out.data_ptr())
+
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            step(B, many)
+            s.synchronize()
+            held = ctx.device_bytes()
+            want = torch.empty((8, 768), device="cuda")
+            step(8, want)
+            s.synchronize()
+            assert ctx.device_bytes() == held
+            got = torch.zeros((8, 768), device="cuda")
+            s.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            graph.capture_begin()
+            step(8, got)
+            graph.capture_end()
+            for i in range(3):
+                got.zero_()
+                graph.replay()
+                s.synchronize()
+                assert torch.equal(got, want), i
+                step(1 + i, many)
+                step(B, many)
+                s.synchronize()
+                assert torch.isfinite(many).all(), i
+
+
 def _prompt_batch(B, V, seed):
     prompts = [synth.prompt(seed + b, n_frames=3 + 4 * b, n_text=4 + b, vocab=V) for b in range(B)]
     n = np.array([p.shape[0] for p in prompts], np.int32)
