@@ -98,16 +98,21 @@ static void release_split(mb_ctx* ctx) {
   if (ctx->split_stream == ctx->stream) ctx->split_claimed = false;
 }
 
+void drop_scratch(mb_ctx* ctx, const char* name) {
+  Scratch& s = ctx->scratch[name];
+  if (!s.ptr) return;
+  (void)hipStreamSynchronize(ctx->stream);
+  (void)hipFree(s.ptr);
+  ctx->device_bytes -= (int64_t)s.bytes;
+  ctx->graph_gen++;
+  s.ptr = nullptr;
+  s.bytes = 0;
+}
+
 void* scratch(mb_ctx* ctx, const char* name, size_t bytes) {
   Scratch& s = ctx->scratch[name];
   if (s.bytes >= bytes && s.ptr) return s.ptr;
-  if (s.ptr) {
-    (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(s.ptr);
-    ctx->device_bytes -= (int64_t)s.bytes;
-    s.ptr = nullptr;
-    s.bytes = 0;
-  }
+  drop_scratch(ctx, name);
   size_t want = bytes < 4096 ? 4096 : bytes;
   ctx->graph_gen++;
   if (hipMalloc(&s.ptr, want) != hipSuccess) {

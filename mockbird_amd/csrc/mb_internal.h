@@ -219,6 +219,7 @@ struct DeviceGuard {
 
 // Device scratch named `name` of at least `bytes`, kept between calls.
 void* scratch(mb_ctx* ctx, const char* name, size_t bytes);
+void drop_scratch(mb_ctx* ctx, const char* name);
 
 // The uploaded tensor `name` if its dims are `dims`; otherwise null, and the
 // first problem is recorded in `missing` ("weight not uploaded: ...").

@@ -239,11 +239,26 @@ int prompt_planes(const mb_ctx* ctx, int64_t M) {
   return M >= kPlanesMinRows3 ? 3 : 0;
 }
 
-// The three-plane weight copies of every global layer.
+// The three-plane weight copies of every global layer, given back.
+void drop_weight_planes(mb_ctx* ctx) {
+  ctx->model.planes = false;
+  for (size_t l = 0; l < ctx->model.layers.size(); l++)
+    for (const char* name : {".attn.3", ".proj.3", ".fc_in.3", ".fc_out.3"})
+      drop_internal(ctx, "#fold/h" + std::to_string(l) + name);
+}
+
+// Makes them.  MB_ERR_NOMEM leaves none behind; the prompt pass then takes the
+// kernels that need none.
 int weight_planes(mb_ctx* ctx) {
   ModelW& m = ctx->model;
   if (m.planes) return MB_OK;
-  for (size_t l = 0; l < m.layers.size(); l++) {
+  // (asked first, so that a full card costs no copies made and dropped a call)
+  size_t room = 0, all = 0;
+  const size_t need = m.layers.size() * ((size_t)D * (QKV + D + 2 * FFN) * 6);
+  MB_HIP(ctx, hipMemGetInfo(&room, &all));
+  if (room < need) return fail(ctx, MB_ERR_NOMEM, "no room for %zu bytes of weight planes", need);
+  int rc = MB_OK;
+  for (size_t l = 0; l < m.layers.size() && !rc; l++) {
     LayerW& w = m.layers[l];
     const std::string key = "#fold/h" + std::to_string(l);
     auto one = [&](const char* name, const float* Wt, int K, int N, const void*& w3) {
@@ -252,15 +267,33 @@ int weight_planes(mb_ctx* ctx) {
       w3 = p;
       return launch_split_w3(ctx, Wt, K, N, p);
     };
-    int rc;
     if ((rc = one(".attn.3", w.attn_wg, D, QKV, w.attn_w3)) ||
         (rc = one(".proj.3", w.proj_wt, D, D, w.proj_w3)) ||
         (rc = one(".fc_in.3", w.fc_in_wg, D, FFN, w.fc_in_w3)) ||
         (rc = one(".fc_out.3", w.fc_out_wt, FFN, D, w.fc_out_w3)))
-      return rc;
+      break;
   }
-  m.planes = true;
-  return MB_OK;
+  if (rc == MB_ERR_NOMEM) drop_weight_planes(ctx);
+  m.planes = rc == MB_OK;
+  return rc;
+}
+
+// The activations of a prompt pass of M rows on `planes` planes.  Three planes
+// take weight copies (510 MB at 12 layers) and activations half as large
+// again; where either does not fit, both are given back and the pass runs on
+// the kernels that need neither (planes = 0), in the memory those need.
+int prompt_activations(mb_ctx* ctx, int64_t M, int& planes, Act& a) {
+  if (planes != 3) return activations(ctx, M, a, planes);
+  const std::string err = ctx->err;
+  int rc = weight_planes(ctx);
+  if (rc == MB_OK) rc = activations(ctx, M, a, planes);
+  if (rc != MB_ERR_NOMEM) return rc;
+  (void)hipGetLastError();
+  ctx->err = err;
+  planes = 0;
+  drop_weight_planes(ctx);
+  for (const char* name : {"act_norm", "act_att", "act_ffn"}) drop_scratch(ctx, name);
+  return activations(ctx, M, a);
 }
 
 // run_layer's prompt form on P planes: each operand's planes are written by
@@ -703,12 +736,8 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
   }
   if ((rc = check_ids(ctx, packed, M))) return rc;
   int planes = prompt_planes(ctx, M);
-  if (planes == 3 && weight_planes(ctx)) {
-    planes = 0;  // no room for the copies: the kernels that need none
-    (void)hipGetLastError();
-  }
   Act a;
-  if ((rc = activations(ctx, M, a, planes))) return rc;
+  if ((rc = prompt_activations(ctx, M, planes, a))) return rc;
   int32_t* d_meta = (int32_t*)scratch(ctx, "prefill_meta", meta.size() * 4);
   float* d_hidden = (float*)scratch(ctx, "hidden", (size_t)B * D * 4);
   if (!d_meta || !d_hidden) return fail(ctx, MB_ERR_NOMEM, "staging allocation failed");

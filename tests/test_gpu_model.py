@@ -693,3 +693,43 @@ def test_large_prompt_batches_equal_single_prompts(kv, weights, voices):
                 assert np.abs(k - k1)[live].max() < 10 * tol and np.abs(v - v1)[live].max() < 10 * tol
         say(f"  max difference {worst:.2e}")
         assert worst < tol
+
+
+@pytest.mark.parametrize("room_mb", [150, 290])
+def test_large_prompts_without_room_for_weight_planes(room_mb):
+    """Large fp32 prompt batches where the card has no room for the weight
+    planes (255 MB at 6 layers), or for them and the activations they take (69
+    MB, 52 without), run in the memory they need without: the same rows within
+    the fp32 bar, nothing kept, no error left behind.  With room again, the
+    bits of a context that had it."""
+    torch = pytest.importorskip("torch")
+    say(f"large prompts in {room_mb} MB")
+    L, V, B, R = 6, 64, 7, 205
+    w = synth.model_weights(n_layers=L, vocab=V, seed=5)
+    g = np.random.default_rng(7)
+    n = np.full(B, R, np.int32)
+    n[3] = 131
+    ids = np.full((B, R, 17), 1024, np.int32)
+    ids[:, :, 0] = g.integers(0, V, size=(B, R))
+    with _ctx(w, L, V, B, 256) as ref:
+        want = ref.prefill(ids, n)
+    with _ctx(w, L, V, B, 256) as ctx:
+        ctx.prefill(ids[:1], n[:1])
+        held = ctx.device_bytes()
+        torch.cuda.empty_cache()
+        filler = []
+        try:
+            for _ in range(3):  # what one large allocation leaves is not exact
+                over = torch.cuda.mem_get_info()[0] - (room_mb << 20)
+                if over > 0:
+                    filler.append(torch.empty(over, dtype=torch.uint8, device="cuda"))
+            for _ in range(2):
+                got = ctx.prefill(ids, n)
+                assert ctx.device_bytes() - held < 60 << 20
+                assert ctx.lib.mb_last_error(ctx.h) == b""
+                assert np.abs(got - want).max() < 1e-4
+                assert not np.array_equal(got, want)  # the other kernels ran
+        finally:
+            del filler
+            torch.cuda.empty_cache()
+        assert np.array_equal(ctx.prefill(ids, n), want)
