@@ -72,6 +72,7 @@ struct CodecState {
   int layer0[kStages] = {};  // first layer (numbered across stages) of each stage
   int slots[kStages] = {};   // ring slots of each stage: context + positions per frame
   std::vector<int64_t> kv_off, sp_off;  // per layer: element offsets in ring_k/v, slot_pos
+  int64_t voice_bytes = 0;  // K and V of one voice's rings, all layers
   void* ring_k = nullptr;
   void* ring_v = nullptr;
   int32_t* slot_pos = nullptr;
@@ -197,6 +198,18 @@ int gemm(mb_ctx* ctx, int epi, const float* A, int64_t lda, const float* W, int 
          const float* bias, float* C, int64_t ldc, int M) {
   return launch_gemm(ctx, epi, A, lda, W, N, K, bias, C, ldc, M, false, nullptr, 0, kCodecGemvRows);
 }
+
+// A window is read once a frame.  Once the rings of a call's voices exceed
+// what the last-level cache (256 MB) keeps of them until the next frame, loads
+// with the streaming hint are the faster ones; below that they lose what it
+// keeps.  Four frames, plain -> hint, at the full depth (24 MB a voice in bf16,
+// 48 in fp32): bf16 4 / 8 / 16 / 32 / 64 / 256 voices 1554 -> 1572, 1630 ->
+// 1620, 1997 -> 1806, 2431 -> 2225, 3263 -> 3037, 8391 -> 8185 us; fp32 1 / 4 /
+// 8 / 12 / 64 / 200 voices 1754 -> 1769, 1818 -> 1820, 2206 -> 1955, 2446 ->
+// 2317, 4753 -> 4618, 13564 -> 13153.  Shallow rings that stay in the cache
+// differ less, either way: 64 voices with windows of 100 slots, hint -> plain,
+// bf16 2098 -> 2083 us, fp32 2366 -> 2383.
+constexpr int64_t kStreamRingBytes = 190000000;
 
 int cancelled(mb_ctx* ctx) {
   if (ctx->cancel.load()) return fail(ctx, MB_ERR_CANCELLED, "cancelled");
@@ -383,6 +396,7 @@ int codec_resolve(mb_ctx* ctx) {
 int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T) {
   CodecState& cs = *ctx->codec;
   const int V = cs.cfg.max_voices;
+  const bool stream = B * cs.voice_bytes >= kStreamRingBytes;
   int rc;
   hipLaunchKernelGGL(k_rvq_accum, dim3((unsigned)(((int64_t)B * kRvq + 255) / 256)), dim3(256), 0,
                      ctx->stream, codes, cs.frame, B, cs.rvq_w, cs.rvq_b, cs.rvq_book, cs.acc);
@@ -429,7 +443,7 @@ int codec_frame(mb_ctx* ctx, int B, const int32_t* codes, float* pcm, int64_t T)
       };
       if ((rc = qkv_proj()) ||
           (rc = launch_window_attention(ctx, ring, B, n, cs.qkv, dense_rows(3 * kD, n), pos, nrow,
-                                        cs.att, dense_rows(kD, n), cs.part)) ||
+                                        cs.att, dense_rows(kD, n), cs.part, stream)) ||
           (rc = x3 ? launch_gemm_x3(ctx, EPI_SCALE_ADD, cs.att, kD, w.o_x, kD, kD, w.s1, cs.x, kD,
                                       M, nullptr, nullptr)
                      : gemm(ctx, EPI_SCALE_ADD, cs.att, kD, w.o, kD, kD, w.s1, cs.x, kD, M)) ||
@@ -505,6 +519,7 @@ extern "C" int mb_codec_init(mb_ctx* ctx, const mb_codec_config* cfg) {
       cs->sp_off.push_back(sp);
       kv += (int64_t)V * kHeads * cs->slots[s] * HD;
       sp += (int64_t)V * cs->slots[s];
+      cs->voice_bytes += (int64_t)2 * kHeads * cs->slots[s] * HD * e;
       cs->n_layers++;
     }
   }

@@ -326,11 +326,13 @@ int launch_prefill_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_
 // into the ring as launch_ring_write writes it, then its query attends.
 // part: room for kWindowPartFloats floats lets few sequences' windows be
 // shared between workgroups; null keeps one workgroup per (sequence, head).
+// stream: the K/V loads carry the streaming hint (windows that the last-level
+// cache will not hold until they are read again).
 constexpr size_t kWindowPartFloats = (size_t)256 * 32 * 68;
 int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                             const float* qkv, const Rows& qkv_rows, const int32_t* pos0,
                             const int32_t* n_rows, float* out, const Rows& out_rows,
-                            float* part = nullptr);
+                            float* part = nullptr, bool stream = false);
 int launch_fill_i32(mb_ctx* ctx, int32_t* p, int64_t n, int32_t value);
 // the first n words of `rows` rows, `stride` words apart
 int launch_fill_rows_i32(mb_ctx* ctx, int32_t* p, int rows, int64_t stride, int64_t n, int32_t value);

@@ -1259,7 +1259,8 @@ int window_splits(int units, int slots) {
 // workgroups, whose states a second launch merges.
 int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_max,
                             const float* qkv, const Rows& qkv_rows, const int32_t* pos0,
-                            const int32_t* n_rows, float* out, const Rows& out_rows, float* part) {
+                            const int32_t* n_rows, float* out, const Rows& out_rows, float* part,
+                            bool stream) {
   if (rows_max < 1 || rows_max > 32)
     return fail(ctx, MB_ERR_ARG, "window attention takes 1..32 rows per sequence, not %d", rows_max);
   if (B > 65535) return fail(ctx, MB_ERR_ARG, "at most 65535 sequences per call");
@@ -1267,14 +1268,6 @@ int launch_window_attention(mb_ctx* ctx, const RingView& ring, int B, int rows_m
   constexpr int NW = kWindowWaves;
   const int S = part ? window_splits(ring.heads * B, ring.C) : 1;
   const dim3 grid((unsigned)ring.heads, (unsigned)B, (unsigned)S);
-  // A window is read once a frame.  Once all layers' rings exceed the last-level
-  // cache (24 MB a voice in bf16, 48 in fp32) loads with the streaming hint are
-  // the faster ones; below that they lose what the cache keeps until the next
-  // frame.  Four frames, plain -> hint: bf16 4 / 8 / 16 / 32 / 64 / 256 voices
-  // 1554 -> 1572, 1630 -> 1620, 1997 -> 1806, 2431 -> 2225, 3263 -> 3037, 8391 ->
-  // 8185 us; fp32 1 / 4 / 8 / 12 / 64 / 200 voices 1754 -> 1769, 1818 -> 1820,
-  // 2206 -> 1955, 2446 -> 2317, 4753 -> 4618, 13564 -> 13153.
-  const bool stream = ring.heads * B * (ring.bf16 ? 2 : 4) >= 64;
   auto go = [&](auto bf_, auto qb_, auto split_, auto st_) {
     constexpr bool BF = decltype(bf_)::value, SP = decltype(split_)::value, ST = decltype(st_)::value;
     constexpr int QB = decltype(qb_)::value;

@@ -166,19 +166,31 @@ def test_codec_shared_windows(B, kv):
     """Few voices: each (voice, head) window is shared between workgroups and
     merged.  Windows just past 2, 2, 4 and 8 workgroups' worth of 16-slot
     groups (8 waves each), decoded from empty rings (workgroups without a
-    group) until stages 2-4 wrap; 17 voices split the long windows only.
-    9 and 17 voices load the window with the streaming hint, 1 and 3 without."""
+    group) until stages 2-4 wrap; 17 voices share every window by two.  The
+    rings stay in the last-level cache: loads without the streaming hint."""
     say(f"codec shared windows, {B} voices, kv={kv}")
-    layers, context = (1, 1, 1, 1), (245, 260, 520, 1030)
+    _check_shared_windows(B, kv, (1, 1, 1, 1), (245, 260, 520, 1030), 40)
+
+
+@pytest.mark.parametrize("B,kv", [(16, mb.MB_KV_BF16), (8, mb.MB_KV_F32)])
+def test_codec_shared_windows_streamed(B, kv):
+    """Shared windows of rings beyond the last-level cache (200 MB: four
+    3248-slot layers), whose loads carry the streaming hint; the shallow
+    stages wrap, stage 4 fills a quarter of its groups."""
+    say(f"codec shared windows streamed, {B} voices, kv={kv}")
+    _check_shared_windows(B, kv, (1, 1, 1, 4), (25, 60, 120, 3248), 24)
+
+
+def _check_shared_windows(B, kv, layers, context, frames):
     watch = sorted({0, B // 2, B - 1})
     w = synth.codec_weights(layers, seed=23)
-    codes = synth.codec_codes(24, 40, B)
+    codes = synth.codec_codes(24, frames, B)
     ora = oracle.CodecOracle(w, len(watch), layers, context, kv_bf16=(kv == mb.MB_KV_BF16))
     want = ora.decode(np.ascontiguousarray(codes[:, watch]))
     with _ctx() as ctx:
         ctx.upload_all(w)
         ctx.codec_init(B, layers, context, kv_dtype=kv)
-        got = np.concatenate([ctx.codec_decode(codes[f:f + 10]) for f in range(0, 40, 10)], axis=2)
+        got = np.concatenate([ctx.codec_decode(codes[f:f + 10]) for f in range(0, frames, 10)], axis=2)
     rel = 2e-5 if kv == mb.MB_KV_F32 else 1e-3
     for i, b in enumerate(watch):
         say(f"  voice {b}: {_close(got[b], want[i], rel, f'voice {b}'):.2e}")
