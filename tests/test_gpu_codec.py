@@ -181,6 +181,16 @@ def test_codec_shared_windows_streamed(B, kv):
     _check_shared_windows(B, kv, (1, 1, 1, 4), (25, 60, 120, 3248), 24)
 
 
+@pytest.mark.parametrize("kv", [mb.MB_KV_F32, mb.MB_KV_BF16])
+def test_codec_windows_shared_by_sixteen(kv):
+    """One voice, windows shared by 2, 2, 4 and 16 workgroups (2100 slots: 134
+    groups of the 128 waves that share them), decoded past the last stage's
+    wrap (67 frames), so every share holds rows and the newest ones move
+    through all of them."""
+    say(f"codec windows shared by sixteen, kv={kv}")
+    _check_shared_windows(1, kv, (1, 1, 1, 1), (245, 260, 520, 2100), 75)
+
+
 def _check_shared_windows(B, kv, layers, context, frames):
     watch = sorted({0, B // 2, B - 1})
     w = synth.codec_weights(layers, seed=23)
