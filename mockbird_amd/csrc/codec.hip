@@ -243,7 +243,7 @@ int gather_cols(mb_ctx* ctx, const std::string& name, const float* src, int K, i
                        dmap, n_dst, dst);
   MB_HIP(ctx, hipGetLastError());
   // the map is read by the launch just queued; keep it until the stream passes it
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   *out = dst;
   return MB_OK;
 }
@@ -384,7 +384,7 @@ int codec_resolve(mb_ctx* ctx) {
                           last ? kLatent : kRvqOut, m, false, &cs.stages[s].out_proj)))
       return rc;
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   ctx->codec_ok = true;
   return MB_OK;
 }
@@ -582,7 +582,7 @@ extern "C" int mb_codec_reset(mb_ctx* ctx, int n, const int32_t* voices) {
       }
     }
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -660,7 +660,7 @@ extern "C" int mb_codec_decode(mb_ctx* ctx, int B, int n_frames, const int32_t* 
   MB_HIP(ctx, hipMemcpyAsync(dc, codes, (size_t)nc * 4, hipMemcpyHostToDevice, ctx->stream));
   if ((rc = mb_codec_decode_dev(ctx, B, n_frames, dc, dp))) return rc;
   MB_HIP(ctx, hipMemcpyAsync(pcm, dp, pcm_bytes, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -678,7 +678,7 @@ extern "C" int mb_codec_read_ring(mb_ctx* ctx, int layer, int voice, float* k, f
   while (s + 1 < kStages && layer >= cs.layer0[s + 1]) s++;
   const int C = cs.slots[s];
   if (slots) *slots = C;
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   const RingView ring = codec_ring(ctx, cs, layer, s);
   const bool bf16 = ring.bf16;
   const size_t e = bf16 ? 2 : 4;

@@ -79,23 +79,34 @@ int hip_fail(mb_ctx* ctx, hipError_t e, const char* what) {
   return fail(ctx, MB_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
-// The context's AttnSplit for a call on its stream: none while that stream is
-// captured (a replay would share it with later calls) or another stream's
-// calls may still be using it.
+// The AttnSplit of a kernel-level attention call: its stream's set, a free one
+// if it has none, else none, and none while the stream is captured (a replay
+// would share it with later calls).  A set goes by the stream's handle: the
+// runtime's hipStreamDestroy waits for the stream's work (43 ms of it, queued
+// before), so a handle that another stream gets later brings none along.
 static AttnSplit claim_split(mb_ctx* ctx) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (ctx->split_claimed && ctx->split_stream != ctx->stream) return {};
   if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return {};
   }
-  ctx->split_claimed = true;
-  ctx->split_stream = ctx->stream;
-  return {ctx->split_part[1], ctx->split_count[1]};
+  int set = 0;
+  for (int i = 1; i < kSplitSets; i++) {
+    if (ctx->split_taken[i] && ctx->split_stream[i] == ctx->stream) return split_set(ctx, i);
+    if (!ctx->split_taken[i] && !set) set = i;
+  }
+  if (!set) return {};
+  ctx->split_taken[set] = true;
+  ctx->split_stream[set] = ctx->stream;
+  return split_set(ctx, set);
 }
-// After the context's stream has been synchronised.
-static void release_split(mb_ctx* ctx) {
-  if (ctx->split_stream == ctx->stream) ctx->split_claimed = false;
+
+hipError_t sync_stream(mb_ctx* ctx) {
+  const hipError_t e = hipStreamSynchronize(ctx->stream);
+  if (e == hipSuccess)
+    for (int i = 1; i < kSplitSets; i++)
+      if (ctx->split_stream[i] == ctx->stream) ctx->split_taken[i] = false;
+  return e;
 }
 
 void drop_scratch(mb_ctx* ctx, const char* name) {
@@ -244,15 +255,13 @@ int mb_create(const mb_config* cfg, mb_ctx** out) {
       e = hipMemcpy(ctx->rope_tab, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice);
       if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMemcpy(rope table)"); break; }
     }
-    e = hipMalloc(&ctx->split_part[0], 2 * (kSplitFloats + kSplitMaxUnits) * 4);
+    e = hipMalloc(&ctx->split_part, kSplitSets * (kSplitFloats + kSplitMaxUnits) * 4);
     if (e != hipSuccess) { rc = hip_fail(ctx, e, "hipMalloc(attention split)"); break; }
-    ctx->split_part[1] = ctx->split_part[0] + kSplitFloats;
-    ctx->split_count[0] = (int32_t*)(ctx->split_part[1] + kSplitFloats);
-    ctx->split_count[1] = ctx->split_count[0] + kSplitMaxUnits;
-    rc = launch_fill_i32(ctx, ctx->split_count[0], 2 * kSplitMaxUnits, 0);
+    ctx->split_count = (int32_t*)(ctx->split_part + kSplitSets * kSplitFloats);
+    rc = launch_fill_i32(ctx, ctx->split_count, kSplitSets * kSplitMaxUnits, 0);
     if (rc) break;
     ctx->device_bytes = 2 * (int64_t)ctx->ring_bytes + slots * 4 + (int64_t)kRopeTab * 32 * 8 +
-                        (int64_t)2 * (kSplitFloats + kSplitMaxUnits) * 4;
+                        (int64_t)kSplitSets * (kSplitFloats + kSplitMaxUnits) * 4;
     // every slot empty; K/V zero so a read of an unwritten slot is well defined
     rc = launch_fill_kv(ctx, ctx->ring_k, (int64_t)(ctx->ring_bytes / kv_elem_bytes(ctx)), 0.f);
     if (rc) break;
@@ -283,7 +292,7 @@ void mb_destroy(mb_ctx* ctx) {
   (void)hipFree(ctx->ring_v);
   (void)hipFree(ctx->slot_pos);
   (void)hipFree(ctx->rope_tab);
-  (void)hipFree(ctx->split_part[0]);
+  (void)hipFree(ctx->split_part);
   for (void* p : {(void*)ctx->local_k, (void*)ctx->local_v, (void*)ctx->local_sp,
                   (void*)ctx->local_pos, (void*)ctx->seen, (void*)ctx->tokens, (void*)ctx->cont})
     (void)hipFree(p);
@@ -306,8 +315,7 @@ void* mb_get_stream(mb_ctx* ctx) { return ctx ? (void*)ctx->stream : nullptr; }
 int mb_synchronize(mb_ctx* ctx) {
   MB_DEVICE_GUARD(ctx);
   if (!ctx) return MB_ERR_ARG;
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  release_split(ctx);
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -337,7 +345,7 @@ int mb_upload_tensor(mb_ctx* ctx, const char* name, const float* data, const int
   }
   DeviceTensor& t = ctx->weights[name];
   if (t.ptr && t.numel != numel) {
-    MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    MB_HIP(ctx, sync_stream(ctx));
     (void)hipFree(t.ptr);
     ctx->device_bytes -= t.numel * 4;
     t.ptr = nullptr;
@@ -356,7 +364,7 @@ int mb_upload_tensor(mb_ctx* ctx, const char* name, const float* data, const int
   ctx->codec_ok = false;
   ctx->graph_gen++;
   MB_HIP(ctx, hipMemcpyAsync(t.ptr, data, (size_t)numel * 4, hipMemcpyHostToDevice, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -379,7 +387,7 @@ int mb_ring_reset(mb_ctx* ctx, int n, const int32_t* seq_ids) {
         if (rc) return rc;
       }
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -398,7 +406,7 @@ int mb_ring_poison(mb_ctx* ctx, int layer, int seq, int n_slots, float sentinel)
     rc = launch_fill_kv(ctx, (char*)ctx->ring_v + off * e, (int64_t)n_slots * HD, sentinel);
     if (rc) return rc;
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -423,7 +431,7 @@ int mb_read_ring(mb_ctx* ctx, int layer, int seq, int slot0, int n, float* k, fl
       MB_HIP(ctx, hipMemcpyAsync(host.data() + (size_t)h * n * HD * e, src + off * e,
                                  (size_t)n * HD * e, hipMemcpyDeviceToHost, ctx->stream));
     }
-    MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    MB_HIP(ctx, sync_stream(ctx));
     // device [head][slot][dim] -> reference [slot][head*64 + dim]
     for (int h = 0; h < H; h++)
       for (int s = 0; s < n; s++)
@@ -442,7 +450,7 @@ int mb_read_ring(mb_ctx* ctx, int layer, int seq, int slot0, int n, float* k, fl
   if (slot_pos) {
     MB_HIP(ctx, hipMemcpyAsync(slot_pos, ctx->slot_pos + slot_base(ctx, layer, seq) + slot0,
                                (size_t)n * 4, hipMemcpyDeviceToHost, ctx->stream));
-    MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    MB_HIP(ctx, sync_stream(ctx));
   }
   return MB_OK;
 }
@@ -487,12 +495,12 @@ int mb_write_ring(mb_ctx* ctx, int layer, int seq, int slot0, int n, const float
       MB_HIP(ctx, hipMemcpyAsync(dst + off * e, host.data() + (size_t)h * n * HD * e,
                                  (size_t)n * HD * e, hipMemcpyHostToDevice, ctx->stream));
     }
-    MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    MB_HIP(ctx, sync_stream(ctx));
   }
   if (slot_pos) {
     MB_HIP(ctx, hipMemcpyAsync(ctx->slot_pos + slot_base(ctx, layer, seq) + slot0, slot_pos,
                                (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
-    MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    MB_HIP(ctx, sync_stream(ctx));
   }
   return MB_OK;
 }
@@ -646,7 +654,7 @@ int mb_ring_write_rows(mb_ctx* ctx, int layer, int B, int rows_max, const float*
                          MB_DT_F32, dense_rows(D, rows_max));
   if (rc) return rc;
   if (q_out) MB_HIP(ctx, hipMemcpyAsync(q_out, d_q, rows * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -669,7 +677,7 @@ int mb_ring_append(mb_ctx* ctx, int layer, int B, const float* qkv, const int32_
                          d_pos, nullptr, q_out ? d_q : nullptr, MB_DT_F32, dense_rows(D, 1));
   if (rc) return rc;
   if (q_out) MB_HIP(ctx, hipMemcpyAsync(q_out, d_q, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -695,8 +703,7 @@ int mb_decode_attention(mb_ctx* ctx, int layer, int B, const float* q, const int
                    (int64_t)max_pos + 1, d_out, dense_rows(D, 1), claim_split(ctx));
   if (rc) return rc;
   MB_HIP(ctx, hipMemcpyAsync(out, d_out, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  release_split(ctx);
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -724,8 +731,7 @@ int mb_append_attend(mb_ctx* ctx, int layer, int B, const float* qkv, const int3
   if (rc) return rc;
   if (q_out) MB_HIP(ctx, hipMemcpyAsync(q_out, d_q, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(out, d_out, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  release_split(ctx);
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -753,7 +759,7 @@ int mb_prefill_attention(mb_ctx* ctx, int layer, int B, int rows_max, const floa
                                 dense_rows(D, rows_max));
   if (rc) return rc;
   MB_HIP(ctx, hipMemcpyAsync(out, d_out, rows * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 

@@ -105,6 +105,22 @@ struct ModelW {
   const void* head_wx[NVQ];
 };
 
+// Workspace of a decode attention whose (sequence, head) units are shared
+// between waves on different CUs (k_attn_unit's MERGE form): per unit
+// kSplitMaxWaves states and a counter that is zero between launches.  Calls
+// that use one must not overlap; with a null `part` every unit is one
+// workgroup's.
+constexpr int kSplitMaxUnits = 192, kSplitMaxWaves = 16;
+constexpr size_t kSplitFloats = (size_t)kSplitMaxUnits * kSplitMaxWaves * PART;
+struct AttnSplit {
+  float* part = nullptr;
+  int32_t* count = nullptr;
+};
+// Sets a context holds: the model's and four streams'.  (An event behind each
+// launch, for any stream to wait for, took 12 layers of one voice from 86 to 135
+// us, as the launch's own stop event to 113.)
+constexpr int kSplitSets = 5;
+
 // Projections with fewer rows than this run with their LayerNorm folded in.
 constexpr int kFoldMaxM = 1024;
 
@@ -133,15 +149,15 @@ struct mb_ctx {
   int32_t* slot_pos = nullptr;
   size_t ring_bytes = 0;  // bytes of ring_k (== ring_v)
 
-  // The AttnSplits (mb_create), first the model's steps', which like their
-  // activations serve one call at a time, then the kernel-level attention
-  // calls'.  The second is used by one stream at a time: the first call after
-  // the last synchronising one claims it (claim_split), calls on other
-  // streams run without.
-  float* split_part[2] = {};
-  int32_t* split_count[2] = {};
-  bool split_claimed = false;
-  hipStream_t split_stream = nullptr;
+  // The AttnSplits (mb_create): set 0 is the model's steps', which like their
+  // activations serve one call at a time, the others the kernel-level
+  // attention calls'.  A stream's first such call takes a free set, which is
+  // the stream's until the context has synchronised it (claim_split,
+  // sync_stream); with none free, and under capture, calls run without.
+  float* split_part = nullptr;
+  int32_t* split_count = nullptr;
+  bool split_taken[mb::kSplitSets] = {};
+  hipStream_t split_stream[mb::kSplitSets] = {};
 
   // RoPE cos/sin for positions [0, kRopeTab): (cos, sin) of pair i at
   // position p in rope_tab[p * 32 + i]; later positions are computed in-kernel.
@@ -219,6 +235,12 @@ struct DeviceGuard {
 
 // Device scratch named `name` of at least `bytes`, kept between calls.
 void* scratch(mb_ctx* ctx, const char* name, size_t bytes);
+// Waits for the context's stream; the AttnSplit set it took is free again.
+hipError_t sync_stream(mb_ctx* ctx);
+// The context's AttnSplit set i.
+inline AttnSplit split_set(const mb_ctx* ctx, int i) {
+  return {ctx->split_part + i * kSplitFloats, ctx->split_count + i * kSplitMaxUnits};
+}
 void drop_scratch(mb_ctx* ctx, const char* name);
 
 // The uploaded tensor `name` if its dims are `dims`; otherwise null, and the
@@ -288,17 +310,6 @@ int launch_ring_write(mb_ctx* ctx, const RingView& ring, int B, int rows_max, co
 // run their attention as per-wave partials merged by the O projection
 // (launch_append_attn_parts, launch_gemv_k_parts).
 constexpr int kPartsMaxSeqs = 8;
-// Workspace of a decode attention whose (sequence, head) units are shared
-// between waves on different CUs (k_attn_unit's MERGE form): per unit
-// kSplitMaxWaves states and a counter that is zero between launches.  Calls
-// that use one must not overlap; with a null `part` every unit is one
-// workgroup's.
-constexpr int kSplitMaxUnits = 192, kSplitMaxWaves = 16;
-constexpr size_t kSplitFloats = (size_t)kSplitMaxUnits * kSplitMaxWaves * PART;
-struct AttnSplit {
-  float* part = nullptr;
-  int32_t* count = nullptr;
-};
 int launch_append_attn_parts(mb_ctx* ctx, const RingView& ring, int B, const float* qkv,
                              const int32_t* pos, int64_t max_valid, float* part, int& nw_out);
 int launch_gemv_k_parts(mb_ctx* ctx, int epi, const float* part, int nwp, const uint16_t* Wk,

@@ -370,7 +370,7 @@ int run_layer(mb_ctx* ctx, const LayerW& w, const RingView& ring, int B, int row
   // attention as per-wave partials merged by the O projection.
   const bool parts = !prefill && gemv && ctx->w_bf16 && pos_const < 0 && B <= kPartsMaxSeqs &&
                      ring.heads == H && ring.window == ring.C;
-  const AttnSplit split = {ctx->split_part[0], ctx->split_count[0]};
+  const AttnSplit split = split_set(ctx, 0);
   static_assert(kPartsMaxSeqs * H <= kSplitMaxUnits && kSplitMaxWaves >= 16, "partials");
   float* const part = split.part;
   int nwp = 0;
@@ -689,7 +689,7 @@ int mb_clear_seen(mb_ctx* ctx, int n, const int32_t* seq_ids) {
       if (rc) return rc;
     }
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -779,7 +779,7 @@ int prefill(mb_ctx* ctx, int B, int rows_max, const int32_t* ids, const int32_t*
       b = e;
     }
   }
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   if (all_hidden)
     for (int b = 0; b < B; b++)
       memset(all_hidden + ((size_t)b * rows_max + n_rows[b]) * D, 0,
@@ -833,7 +833,7 @@ int mb_decode_step(mb_ctx* ctx, int B, const int32_t* rows17, const int32_t* pos
   MB_HIP(ctx, hipMemcpyAsync(d_pos, pos, (size_t)B * 4, hipMemcpyHostToDevice, ctx->stream));
   if ((rc = decode_step(ctx, B, d_rows, d_pos, max_pos, d_hidden))) return rc;
   MB_HIP(ctx, hipMemcpyAsync(hidden, d_hidden, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -851,7 +851,7 @@ int mb_local_frame(mb_ctx* ctx, int B, const float* hidden, int32_t* codes, int3
   if ((rc = local_frame(ctx, B, d_hidden, d_out, d_out + (size_t)B * NVQ, nullptr))) return rc;
   MB_HIP(ctx, hipMemcpyAsync(codes, d_out, (size_t)B * NVQ * 4, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(cont, d_out + (size_t)B * NVQ, (size_t)B * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -870,7 +870,7 @@ int mb_local_steps(mb_ctx* ctx, int B, const float* hidden, int max_step, float*
   Act a;
   if ((rc = local_steps(ctx, B, d_hidden, max_step, false, a))) return rc;
   MB_HIP(ctx, hipMemcpyAsync(out, a.norm, (size_t)B * D * 4, hipMemcpyDeviceToHost, ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -903,7 +903,7 @@ int mb_local_logits(mb_ctx* ctx, int B, const float* hidden, const int32_t* code
   MB_HIP(ctx, hipMemcpyAsync(text2, d_text, (size_t)B * 2 * 8, hipMemcpyDeviceToHost, ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(logits, d_logits, (size_t)B * NVQ * CODES * 4, hipMemcpyDeviceToHost,
                              ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 
@@ -1037,7 +1037,7 @@ int mb_decode_frames(mb_ctx* ctx, int B, int n_frames, float* hidden, int32_t* p
                              ctx->stream));
   MB_HIP(ctx, hipMemcpyAsync(cont, d_cont, (size_t)n_frames * B * 4, hipMemcpyDeviceToHost,
                              ctx->stream));
-  MB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  MB_HIP(ctx, sync_stream(ctx));
   return MB_OK;
 }
 

@@ -395,9 +395,7 @@ def test_units_shared_between_waves(name, kv, B, C):
     """Few units over windows of many batches: each (query, head) unit is
     shared by up to 16 one-wave workgroups and merged by the last.  Windows
     of one slot (waves without a batch), part full and wrapped, a strided
-    output; the same bits on every call, within fp32 rounding (1e-6 of O(1)
-    outputs: sums of up to 1030 weights in another order) of the same call on
-    a stream that does not hold the workspace."""
+    output; the same bits on every call and on a second stream."""
     torch = pytest.importorskip("torch")
     say(f"shared units kv={name} B={B} C={C}")
     rng = np.random.default_rng([B, C])
@@ -425,17 +423,62 @@ def test_units_shared_between_waves(name, kv, B, C):
                                  out[3].data_ptr(), out_stride=832)
         torch.cuda.synchronize()
         other = torch.cuda.Stream()
-        ctx.set_stream(other.cuda_stream)  # the workspace still belongs to the first stream
+        ctx.set_stream(other.cuda_stream)
         ctx.append_attend_dev(0, B, x.data_ptr(), p.data_ptr(), int(max(pos.max(), C)),
                               out[4].data_ptr(), out_stride=832)
         other.synchronize()
         got = out.cpu().numpy()
         _check_ring(ctx, ring, 0, range(B))
-    for i in range(1, 4):
+    for i in range(1, 5):
         assert np.array_equal(got[i], got[0]), i
     assert not got[:, :, 768:].any()
-    assert np.abs(got[4] - got[0]).max() < 1e-6
     assert np.abs(got[0, :, :768] - want).max() < (2e-6 if kv == mb.MB_KV_F32 else 1e-4)
+
+
+@pytest.mark.parametrize("name,kv", KV)
+def test_shared_units_on_several_streams(name, kv):
+    """Four streams a context has not synchronised have a workspace each, so
+    overlapping calls give one another's bits; a fifth stream's calls run
+    without, within fp32 rounding (1e-6 of O(1) outputs: sums of 1000 weights in
+    another order), until the context synchronises one of the four.  A stream
+    synchronised by the caller alone keeps its workspace when the context
+    comes back to it."""
+    torch = pytest.importorskip("torch")
+    say(f"shared units on streams kv={name}")
+    B, C = 2, 1000
+    rng = np.random.default_rng(93)
+    pos = np.array([999, 600], np.int32)
+    dev = torch.device("cuda")
+    with mb.Context(n_layers=1, capacity=C, max_seqs=B, max_rows=1, kv_dtype=kv) as ctx:
+        for b in range(B):
+            k, v = (rng.standard_normal((C, 768)).astype(np.float32) for _ in range(2))
+            ctx.write_ring(0, b, 0, k, v, np.arange(C, dtype=np.int32))
+        q = torch.from_numpy(rng.standard_normal((B, 768)).astype(np.float32)).to(dev)
+        p = torch.from_numpy(pos).to(dev)
+        streams = [torch.cuda.Stream() for _ in range(5)]
+        out = torch.zeros((5, 20, B, 768), device=dev)
+        torch.cuda.synchronize()
+
+        def run(i, j):
+            ctx.set_stream(streams[i].cuda_stream)
+            ctx.decode_attention_dev(0, B, q.data_ptr(), p.data_ptr(), C - 1, out[i, j].data_ptr())
+
+        for j in range(20):
+            for i in range(4):
+                run(i, j)
+        run(4, 0)
+        torch.cuda.synchronize()
+        run(2, 0)  # still its own
+        streams[2].synchronize()
+        assert torch.equal(out[:4], out[:1, :1].expand(4, 20, B, 768))
+        plain = out[4, 0].clone()
+        assert (plain - out[0, 0]).abs().max() < 1e-6
+        if kv == mb.MB_KV_F32:  # (bf16: 16 waves of one batch either way)
+            assert not torch.equal(plain, out[0, 0])
+        ctx.synchronize()  # the third stream's workspace
+        run(4, 1)
+        torch.cuda.synchronize()
+        assert torch.equal(out[4, 1], out[0, 0])
 
 
 @pytest.mark.parametrize("name,kv", KV)
