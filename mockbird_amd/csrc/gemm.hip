@@ -412,12 +412,12 @@ __device__ __forceinline__ void stream_finish(f32x4_t (&acc)[MI][4], float (&sx)
 // -- which requires the workgroup to see the whole row (S == 1, K == 768).
 //
 // ALT with tiles of 32 rows and more (PLANES): the products on the bf16
-// matrix unit.  A wave splits the A rows and
-// W columns it holds into three exact bf16 planes each (planes.h) and sums the
-// six plane products above 2^-24 in fp32: per 16 x 16 x 32 block 6 MFMAs of 16
-// cycles in place of 8 of 32.  Its error against float64 is the smaller one
-// (768-deep 2.5e-7 -> 2.1e-7, 3072-deep 5.0e-7 -> 4.3e-7 relative: fewer
-// roundings of the running sum).  stream_planes says where it is taken.
+// matrix unit.  A wave splits the A rows and W columns it holds into three
+// exact bf16 planes each (planes.h) and sums six plane products in fp32, all
+// but 2^-24 of the product: per 16 x 16 x 32 block 6 MFMAs of 16 cycles in
+// place of 8 of 32.  Its error against float64 is the smaller one (768-deep
+// 2.5e-7 -> 2.0e-7, 3072-deep 5.0e-7 -> 4.2e-7 relative: fewer roundings of
+// the running sum).  stream_planes says where it is taken.
 //
 // ALT with 16-row tiles (the codec's, launch_gemm's gemv_rows): the two stages
 // are summed apart, with half as many roundings of a running sum.  That keeps
@@ -786,8 +786,8 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ p
 // tiles of 32 rows and more over at least 512 k.  There the fp32
 // matrix rate bounds the loop; smaller tiles wait for W, and the splits only
 // add to that.  fp32 MFMA -> planes, us: 2304 x 768 at 281 / 500 / 1000 rows
-// 12.3 -> 10.7, 34.4 -> 24.7, 57.7 -> 36.8 (48- and 64-row tiles); 768 x 3072
-// at 100 / 281 / 1000 rows 11.3 -> 10.9, 17.5 -> 15.8, 39.6 -> 31.5 (32-row
+// 12.3 -> 10.9, 34.4 -> 25.1, 57.7 -> 37.6 (48- and 64-row tiles); 768 x 3072
+// at 100 / 281 / 1000 rows 11.3 -> 11.0, 17.5 -> 16.7, 39.6 -> 33.0 (32-row
 // ones); 256 x 256 at 2048 rows 4.9 -> 5.2, 768 x 768 at 64 rows 5.5 -> 6.1
 // (16-row tiles).  Over 256 k a wave has two blocks to split for: four
 // codec frames of 40 / 64 / 100 voices took 4087 / 4601 / 7348 us with planes in

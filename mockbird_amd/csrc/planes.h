@@ -3,11 +3,12 @@
 //  - three planes (split3): x = h + m + l exactly.  h = bf16(x) and m =
 //    bf16(x - h), rounded to nearest even: the remainders are exact and of
 //    either sign, |m| <= 2^-8 |x| and |l| <= 2^-17 |x|, and l has 7 bits at
-//    most.  Below 2^-110 the low plane may be denormal.  A magnitude that
-//    rounds past the largest bf16 (above (2 - 2^-8) 2^127) has no h: its
-//    planes, as an infinity's, give NaN, and kernels that split their operands
-//    themselves take such sums again in fp32; planes that are stored (SAT)
-//    stop h at the largest bf16, which leaves the sum exact.
+//    most.  (bf16 ends at 2^-133: of values below 2^-110, whose bits go on
+//    below it, that much is lost.)  A magnitude that rounds past the largest
+//    bf16 (above (2 - 2^-8) 2^127) has no h: its planes, as an infinity's, give
+//    NaN, and kernels that split their operands themselves take such sums
+//    again in fp32; planes that are stored (SAT) stop h at the largest bf16,
+//    which leaves the sum exact.
 //  - two planes (split2): h = bf16(x), l = bf16(x - h), rounded to nearest
 //    even: x to within about 2^-17.
 #pragma once

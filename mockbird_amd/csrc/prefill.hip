@@ -505,8 +505,9 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
 // MFMAs of 16 cycles and one of two fp32 operands six, where
 // v_mfma_f32_16x16x4f32 takes eight of 32.  The fp32 matrix rate bounded the
 // kernel that used it.  The error against float64 is no larger than with fp32
-// products (1 x 281 rows, fp32 ring 2.5e-7 -> 2.3e-7 relative; bf16 ring
-// 3.3e-7 -> 2.8e-7): the sums are fp32 either way, in fewer roundings.
+// products (1 x 281 rows, fp32 ring 2.5e-7 -> 2.2e-7 relative; bf16 ring
+// 3.3e-7 -> 2.8e-7): the sums are fp32 either way, in fewer roundings.  Rows
+// whose sums are not finite are taken again with fp32 products.
 //
 // A workgroup is 64 query rows of one (sequence, head), 16 per wave.  K/V
 // tiles of KS slots pass through registers into one of two LDS buffers (fp32
@@ -515,8 +516,8 @@ __global__ __launch_bounds__(64 * NW, 3 * NW / 4) void k_flash_bf16(
 // 32 for fp32 ones, whose three planes fill the same 48 KB twice over; 64
 // fp32 slots (one workgroup per CU) took 98 us against 72 at 16 x 512 rows.
 // Also slower: 32 rows per wave (1 x 281 / 16 x 512 / 48 x 64..400 rows with
-// the ring write, fp32 ring 22.1 / 74.0 / 99.8 us against 17.5 / 71.6 / 92.8,
-// bf16 15.8 / 51.0 / 70.4 against 12.7 / 48.4 / 63.5: fewer workgroups, more
+// the ring write, fp32 ring 22.1 / 74.0 / 99.8 us against 17.4 / 71.1 / 91.2,
+// bf16 15.8 / 51.0 / 70.4 against 12.8 / 47.9 / 62.9: fewer workgroups, more
 // registers), two waves per workgroup (20.3 / 96.3 / 121.1 us, fp32), and
 // k_flash_bf16's snake order (equal).  With the fp32 MFMA kernel the same
 // calls took 28.3 / 109.3 / 130.6 us (fp32) and 29.1 / 106.2 / 121.7 (bf16).
