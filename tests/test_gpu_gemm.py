@@ -129,6 +129,29 @@ def test_linear_plane_products_one_by_one(ctx, M, N, K):
     assert worst < 3.1
 
 
+def test_linear_planes_values_above_the_largest_bf16(ctx):
+    """Finite values that round past the largest bf16 have no planes either and
+    take their tiles in fp32: the outputs stay finite, within the roundings of
+    K products (K 2^-24 of the sum of their sizes)."""
+    torch = pytest.importorskip("torch")
+    say("linear planes: values above the largest bf16")
+    M, N, K = 281, 2304, 768
+    g = np.random.default_rng(78)
+    A = g.standard_normal((M, K), dtype=np.float32)
+    W = g.standard_normal((K, N), dtype=np.float32) * np.float32(1e-3)
+    A[5, 3], A[70, 700] = 3.4e38, -3.4e38
+    W[100, 9], A[:, 100] = 3.4e38, A[:, 100] * np.float32(1e-3)
+    dev = torch.device("cuda")
+    ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+    tA, tW = torch.from_numpy(A).to(dev), torch.from_numpy(W).to(dev)
+    tC = torch.zeros((M, N), device=dev)
+    ctx.linear_dev(M, N, K, tA.data_ptr(), K, tW.data_ptr(), None, tC.data_ptr(), N)
+    torch.cuda.synchronize()
+    want = tA.double() @ tW.double()
+    size = tA.double().abs() @ tW.double().abs()
+    assert bool(((tC.double() - want).abs() <= K * 2.0 ** -24 * size).all())
+
+
 def test_linear_planes_keep_infinities_and_nan(ctx):
     """An infinity has no planes: the tile that holds one is taken in fp32, so
     infinities, their NaN sums and the finite rows beside them are what fp32
